@@ -10,9 +10,9 @@
 //
 // namsa_build_slices: the reference kernel (namsa/potential_kernels.cu:5-60)
 // lets every pixel thread scan every site of its slice, O(N^2 S A).  Here a
-// workgroup owns a 16x64 pixel tile of one slice, streams that slice's sites
-// through LDS 256 at a time, keeps (in site order, by ballot compaction) only
-// the sites whose clipped footprint overlaps the tile, and accumulates table
+// workgroup owns a tile of one slice (64 x 64 pixels, or 16 x 16 for small
+// launches), streams that slice's sites through LDS, keeps (in site order, by
+// ballot compaction) only those whose clipped footprint overlaps the tile, and accumulates table
 // values for its pixels in float32 in site order; exp(i sigma V) with the NaN
 // guard of potential_kernels.cu:48-57 is fused into the store.
 #include "common.hpp"
@@ -88,96 +88,271 @@ atomic_tables_kernel(const double* __restrict__ params, int Py, int Px, int os, 
 }
 
 // ------------------------------------------------------------------ slice builder
-constexpr int kTileH = 16;
-constexpr int kTileW = 64;
 constexpr int kSliceThreads = 256;
-constexpr int kPxPerThread = kTileH * kTileW / kSliceThreads;  // 4
+constexpr int kWaves = kSliceThreads / 64;
 
+// A site as the accumulation reads it: its table value at pixel (row, col) is
+// tables[base + row * Px + col], for rows [r_lo, r_lo + rows) and columns
+// [c_lo, c_lo + cols).
 struct SiteBox {
-  int z, y0, r_lo, r_hi, x0, c_lo, c_hi;
+  long long base;
+  int r_lo, rows, c_lo, cols;
+  __device__ __forceinline__ void set(long long b, int r, int nr, int c, int nc) {
+    base = b;
+    r_lo = r;
+    rows = nr;
+    c_lo = c;
+    cols = nc;
+  }
 };
 
+// The sites of one slice in order, K per thread at a time: scan() keeps those
+// whose clipped footprint overlaps the tile, in site order, in list[0, total).
+// The next chunk's sites are loaded before the current one is used.
+template <int K>
+struct SiteScan {
+  static constexpr int kChunk = K * kSliceThreads;
+  const int* __restrict__ sites;
+  int nZ, Py, Px, Ny, Nx, end, next;
+  int z[K], yc[K], xc[K];
+
+  __device__ __forceinline__ void fetch() {
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      const int i = next + j * kSliceThreads + static_cast<int>(threadIdx.x);
+      z[j] = -1;
+      if (i < end) {
+        z[j] = sites[3LL * i];
+        yc[j] = sites[3LL * i + 1];
+        xc[j] = sites[3LL * i + 2];
+      }
+    }
+    next += kChunk;
+  }
+
+  // Workgroup-wide: returns the number of boxes in list, which `pad` empty ones
+  // follow (barriers inside).
+  template <class Box>
+  __device__ __forceinline__ int scan(Box* list, int pad, int (*wave_count)[kWaves], int ty0, int th, int tx0, int tw) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    bool hit[K];
+    Box bx[K];
+    int rank[K];
+    __syncthreads();  // the previous chunk's list has been read
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      const int y0 = static_cast<int>(rintf(float(yc[j]) - Py * 0.5f));
+      const int y1 = static_cast<int>(rintf(float(yc[j]) + Py * 0.5f));
+      const int x0 = static_cast<int>(rintf(float(xc[j]) - Px * 0.5f));
+      const int x1 = static_cast<int>(rintf(float(xc[j]) + Px * 0.5f));
+      const int r_lo = max(y0, 0), r_hi = min(min(y1, Ny), y0 + Py);
+      const int c_lo = max(x0, 0), c_hi = min(min(x1, Nx), x0 + Px);
+      bx[j].set((static_cast<long long>(z[j]) * Py - y0) * Px - x0, r_lo, r_hi - r_lo, c_lo, c_hi - c_lo);
+      hit[j] = z[j] >= 0 && z[j] < nZ && r_lo < r_hi && c_lo < c_hi && r_lo < ty0 + th && r_hi > ty0 &&
+               c_lo < tx0 + tw && c_hi > tx0;
+      // order-preserving compaction: rank = hits in lower lanes, then in lower waves and rounds
+      const unsigned long long ballot = __ballot(hit[j]);
+      rank[j] = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(ballot >> 32),
+                                          __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(ballot), 0));
+      if (lane == 0) wave_count[j][wave] = __popcll(ballot);
+    }
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        if (w == wave && hit[j]) list[total + rank[j]] = bx[j];
+        total += wave_count[j][w];
+      }
+    total = __builtin_amdgcn_readfirstlane(total);
+    if (static_cast<int>(threadIdx.x) < pad) list[total + threadIdx.x] = Box{};
+    if (next < end) fetch();
+    __syncthreads();
+    return total;
+  }
+};
+
+// V or t = exp(i sigma V) of one pixel, NaN components of t replaced by 1.
+template <bool POT>
+__device__ __forceinline__ void put_pixel(float acc, float sigma, long long o, float2* t_out, float* v_out) {
+  if constexpr (POT) {
+    v_out[o] = acc;
+  } else {
+    float sn, cs;
+    sincosf(acc * sigma, &sn, &cs);
+    if (isnan(cs)) cs = 1.0f;
+    if (isnan(sn)) sn = 1.0f;
+    t_out[o] = make_float2(cs, sn);
+  }
+}
+
+// Tile of 64 x 64 pixels, 16 rows of 64 columns per wavefront, for launches
+// with enough tiles.  The sums are bound by instructions and address
+// generation, so a site's box is decoded once per 16 rows, into scalar
+// registers: inside the columns of the box a row is then one read (scalar row
+// address, one lane offset) and one add, and all 16 reads are issued before
+// the first sum.  Sums run in site order in float32, as in the narrow kernel,
+// so both give the same bits.  Against 16 x 64 tiles of 4 rows per wavefront
+// that took one site at a time, t of 512^2 x 150 slices (491 sites each):
+// 321 -> 162 us, 1.9 TB/s written; 2048^2 x 60 (3930 sites): 2.10 -> 1.02 ms.
 // POT: write the projected potential V (float) instead of t = exp(i sigma V).
+constexpr int kWideRows = 16;
+
 template <bool POT>
 __global__ void __launch_bounds__(kSliceThreads)
-build_slices_kernel(const float* __restrict__ tables, int nZ, int Py, int Px,
-                    const int* __restrict__ sites,
-                    const int* __restrict__ offsets, int Ny, int Nx, float sigma,
-                    float2* __restrict__ t_out, float* __restrict__ v_out) {
-  __shared__ SiteBox list[kSliceThreads];
-  __shared__ int wave_count[kSliceThreads / 64];
-
+build_slices_wide_kernel(const float* __restrict__ tables, int nZ, int Py, int Px, const int* __restrict__ sites,
+                         const int* __restrict__ offsets, int Ny, int Nx, float sigma, float2* __restrict__ t_out,
+                         float* __restrict__ v_out) {
+  using Scan = SiteScan<1>;
+  __shared__ SiteBox list[Scan::kChunk];
+  __shared__ int wave_count[1][kWaves];
+  const auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   const int s = blockIdx.z;
-  const int ty0 = blockIdx.y * kTileH, tx0 = blockIdx.x * kTileW;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int col = tx0 + lane;
-  float acc[kPxPerThread];
+  const int ty0 = blockIdx.y * kWaves * kWideRows, tx0 = blockIdx.x * 64;
+  const int row0 = ty0 + uni(threadIdx.x >> 6) * kWideRows;
+  const int col = tx0 + (threadIdx.x & 63);
+  float acc[kWideRows];
 #pragma unroll
-  for (int k = 0; k < kPxPerThread; ++k) acc[k] = 0.0f;
+  for (int k = 0; k < kWideRows; ++k) acc[k] = 0.0f;
 
-  const int beg = offsets[s], end = offsets[s + 1];
-  for (int base = beg; base < end; base += kSliceThreads) {
-    const int i = base + threadIdx.x;
-    bool hit = false;
-    SiteBox bx{};
-    if (i < end) {
-      const int z = sites[3 * i], yc = sites[3 * i + 1], xc = sites[3 * i + 2];
-      bx.z = z;
-      bx.y0 = static_cast<int>(rintf(float(yc) - Py * 0.5f));
-      const int y1 = static_cast<int>(rintf(float(yc) + Py * 0.5f));
-      bx.x0 = static_cast<int>(rintf(float(xc) - Px * 0.5f));
-      const int x1 = static_cast<int>(rintf(float(xc) + Px * 0.5f));
-      bx.r_lo = max(bx.y0, 0);
-      bx.r_hi = min(min(y1, Ny), bx.y0 + Py);
-      bx.c_lo = max(bx.x0, 0);
-      bx.c_hi = min(min(x1, Nx), bx.x0 + Px);
-      hit = z >= 0 && z < nZ && bx.r_lo < bx.r_hi && bx.c_lo < bx.c_hi && bx.r_lo < ty0 + kTileH &&
-            bx.r_hi > ty0 && bx.c_lo < tx0 + kTileW && bx.c_hi > tx0;
-    }
-    // order-preserving compaction: rank = hits in lower lanes + hits in lower waves
-    const unsigned long long ballot = __ballot(hit);
-    const int rank_in_wave = __builtin_amdgcn_mbcnt_hi(
-        static_cast<unsigned>(ballot >> 32),
-        __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(ballot), 0));
-    if (lane == 0) wave_count[wave] = __popcll(ballot);
-    __syncthreads();
-    int offset = 0, total = 0;
+  Scan scan{sites, nZ, Py, Px, Ny, Nx, offsets[s + 1], offsets[s]};
+  if (scan.next < scan.end) {
+    scan.fetch();
+    for (int base = offsets[s]; base < scan.end; base += Scan::kChunk) {
+      const int total = scan.scan(list, 0, wave_count, ty0, kWaves * kWideRows, tx0, 64);
+      for (int e = 0; e < total; ++e) {
+        const SiteBox& b = list[e];
+        const int dr = row0 - uni(b.r_lo), rows = uni(b.rows);
+        if (dr <= -kWideRows || dr >= rows) continue;
+        if (static_cast<unsigned>(col - b.c_lo) >= static_cast<unsigned>(b.cols)) continue;
+        const long long at = (static_cast<long long>(uni(static_cast<int>(b.base >> 32))) << 32) |
+                             static_cast<unsigned>(uni(static_cast<int>(b.base)));
+        const float* line = tables + at + static_cast<long long>(row0) * Px;
+        float v[kWideRows];
+        if (dr >= 0 && dr + kWideRows <= rows) {
 #pragma unroll
-    for (int w = 0; w < kSliceThreads / 64; ++w) {
-      if (w < wave) offset += wave_count[w];
-      total += wave_count[w];
-    }
-    if (hit) list[offset + rank_in_wave] = bx;
-    __syncthreads();
-    for (int e = 0; e < total; ++e) {
-      const SiteBox b = list[e];
-      if (col < b.c_lo || col >= b.c_hi) continue;
-      const float* tab = tables + static_cast<long long>(b.z) * Py * Px + (col - b.x0);
+          for (int k = 0; k < kWideRows; ++k) v[k] = (line + static_cast<long long>(k) * Px)[static_cast<unsigned>(col)];
+        } else {  // rows outside the box add +0 to a sum that is never -0
 #pragma unroll
-      for (int k = 0; k < kPxPerThread; ++k) {
-        const int row = ty0 + wave + 4 * k;
-        if (row >= b.r_lo && row < b.r_hi) acc[k] += tab[(row - b.y0) * Px];
+          for (int k = 0; k < kWideRows; ++k) {
+            v[k] = 0.0f;
+            if (static_cast<unsigned>(dr + k) < static_cast<unsigned>(rows)) v[k] = (line + static_cast<long long>(k) * Px)[static_cast<unsigned>(col)];
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < kWideRows; ++k) acc[k] += v[k];
       }
     }
-    __syncthreads();
   }
-
   const long long plane = static_cast<long long>(Ny) * Nx;
+  // one copy of the sine and cosine: unrolled over the rows they take 89
+  // registers (5 wavefronts per SIMD)
+#pragma unroll 1
+  for (int k = 0; k < kWideRows; ++k) {
+    if (row0 + k < Ny && col < Nx)
+      put_pixel<POT>(acc[0], sigma, s * plane + static_cast<long long>(row0 + k) * Nx + col, t_out, v_out);
 #pragma unroll
-  for (int k = 0; k < kPxPerThread; ++k) {
-    const int row = ty0 + wave + 4 * k;
-    if (row < Ny && col < Nx) {
-      if constexpr (POT) {
-        v_out[s * plane + static_cast<long long>(row) * Nx + col] = acc[k];
-        continue;
+    for (int j = 0; j + 1 < kWideRows; ++j) acc[j] = acc[j + 1];
+  }
+}
+
+// Tile of 16 x 16 pixels, one per thread, for launches too small for the wide
+// one (a single projected plane, short stacks of small grids).  There the
+// chain of reads of a pixel is what takes the time: boxes and table values
+// are read kNarrowBatch sites ahead of the sums, without conditions: a pixel
+// outside a site's box reads past the end of the tables' buffer, which gives
+// +0, and adds it to a sum that is never -0.  The list ends in empty boxes, so
+// batches need no remainder.  Offsets into the tables are 32-bit and box sides
+// 16-bit (the launcher checks).  One 256^2 plane of 24,573 sites: 2010 us in
+// 16 x 64 tiles one site at a time, 175 us now.
+// K: sites per thread and scan; 4 for one long list (a scan's barriers are
+// then paid once per 1024 sites), 1 for many short ones.
+constexpr int kNarrow = 16, kNarrowBatch = 8;
+
+struct alignas(16) NarrowBox {  // one LDS read
+  unsigned base;
+  int r_lo, c_lo;
+  unsigned size;  // columns << 16 | rows
+  __device__ __forceinline__ void set(long long b, int r, int nr, int c, int nc) {
+    base = static_cast<unsigned>(b);
+    r_lo = r;
+    c_lo = c;
+    size = static_cast<unsigned>(nc) << 16 | static_cast<unsigned>(nr);
+  }
+};
+
+template <bool POT, int K>
+__global__ void __launch_bounds__(kSliceThreads)
+build_slices_narrow_kernel(const float* __restrict__ tables, int nZ, int Py, int Px, const int* __restrict__ sites,
+                           const int* __restrict__ offsets, int Ny, int Nx, float sigma, float2* __restrict__ t_out,
+                           float* __restrict__ v_out) {
+  using Scan = SiteScan<K>;
+  __shared__ NarrowBox list[Scan::kChunk + 2 * kNarrowBatch];
+  __shared__ int wave_count[K][kWaves];
+  const int s = blockIdx.z;
+  const int ty0 = blockIdx.y * kNarrow, tx0 = blockIdx.x * kNarrow;
+  const int row = ty0 + static_cast<int>(threadIdx.x / kNarrow), col = tx0 + static_cast<int>(threadIdx.x % kNarrow);
+  const unsigned pixel = static_cast<unsigned>(row) * static_cast<unsigned>(Px) + static_cast<unsigned>(col);
+  const unsigned table_bytes = static_cast<unsigned>(nZ) * Py * Px * 4u;
+  const auto buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(tables), 0, static_cast<int>(table_bytes),
+                                                     0x00020000);
+  float acc = 0.0f;
+  Scan scan{sites, nZ, Py, Px, Ny, Nx, offsets[s + 1], offsets[s]};
+  if (scan.next < scan.end) {
+    scan.fetch();
+    for (int base = offsets[s]; base < scan.end; base += Scan::kChunk) {
+      const int total = scan.scan(list, 2 * kNarrowBatch, wave_count, ty0, kNarrow, tx0, kNarrow);
+      float v[kNarrowBatch], w[kNarrowBatch];
+      const auto read = [&](int e, float(&out)[kNarrowBatch]) {
+        NarrowBox b[kNarrowBatch];
+#pragma unroll
+        for (int u = 0; u < kNarrowBatch; ++u) b[u] = list[e + u];
+        // no short-circuit: a branch per site would wait for its LDS read
+#pragma unroll
+        for (int u = 0; u < kNarrowBatch; ++u) {
+          const bool in = (static_cast<unsigned>(row - b[u].r_lo) < (b[u].size & 0xffffu)) &
+                          (static_cast<unsigned>(col - b[u].c_lo) < (b[u].size >> 16));
+          const unsigned at = (b[u].base + pixel) * 4u;
+          out[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buf, in ? at : table_bytes, 0, 0));
+        }
+      };
+      read(0, v);
+      for (int e = 0; e < total; e += kNarrowBatch) {
+        read(e + kNarrowBatch, w);
+#pragma unroll
+        for (int u = 0; u < kNarrowBatch; ++u) {
+          acc += v[u];
+          v[u] = w[u];
+        }
       }
-      float sn, cs;
-      sincosf(acc[k] * sigma, &sn, &cs);
-      if (isnan(cs)) cs = 1.0f;
-      if (isnan(sn)) sn = 1.0f;
-      t_out[s * plane + static_cast<long long>(row) * Nx + col] = make_float2(cs, sn);
     }
   }
+  if (row < Ny && col < Nx)
+    put_pixel<POT>(acc, sigma, s * (static_cast<long long>(Ny) * Nx) + static_cast<long long>(row) * Nx + col, t_out,
+                   v_out);
+}
+
+template <bool POT>
+int launch_build(const float* tables, int nZ, int Py, int Px, const int* sites, const int* offsets, int S, int Ny,
+                 int Nx, float sigma, float2* t_out, float* v_out, hipStream_t st) {
+  const auto tiles = [](int n, int t) { return static_cast<unsigned>((n + t - 1) / t); };
+  const dim3 wide(tiles(Nx, 64), tiles(Ny, kWaves * kWideRows), S);
+  const dim3 narrow(tiles(Nx, kNarrow), tiles(Ny, kNarrow), S);
+  // Wide from 4 workgroups per CU up (256^2 x 50 slices, 3.1 per CU: equal;
+  // 128^2 x 60, 0.9 per CU: 14 us wide, 10 narrow; one 256^2 plane, 16
+  // workgroups: 1014 and 95), or where narrow's offsets or grid end.
+  if (static_cast<long long>(wide.x) * wide.y * S >= 4LL * device_cu_count() || narrow.y > 65535 ||
+      static_cast<long long>(nZ) * Py * Px >= (1LL << 29) || Py > 65535 || Px > 65535)
+    hipLaunchKernelGGL(build_slices_wide_kernel<POT>, wide, dim3(kSliceThreads), 0, st, tables, nZ, Py, Px, sites,
+                       offsets, Ny, Nx, sigma, t_out, v_out);
+  else if (S > 1)
+    hipLaunchKernelGGL((build_slices_narrow_kernel<POT, 1>), narrow, dim3(kSliceThreads), 0, st, tables, nZ, Py, Px, sites,
+                       offsets, Ny, Nx, sigma, t_out, v_out);
+  else
+    hipLaunchKernelGGL((build_slices_narrow_kernel<POT, 4>), narrow, dim3(kSliceThreads), 0, st, tables, nZ, Py, Px, sites,
+                       offsets, Ny, Nx, sigma, t_out, v_out);
+  return check_hip(hipGetLastError(), "build_slices_kernel launch");
 }
 
 // ------------------------------------------------- sampled 3D potentials
@@ -257,10 +432,8 @@ int namsa_build_slices(const float* tables, int nZ, int Py, int Px, const int* s
     return fail(kErrArg, "namsa_build_slices: bad arguments");
   if (S == 0) return kOk;
   if (S > 65535) return fail(kErrArg, "namsa_build_slices: S=%d exceeds the grid z limit", S);
-  dim3 grid((Nx + kTileW - 1) / kTileW, (Ny + kTileH - 1) / kTileH, S);
-  hipLaunchKernelGGL(build_slices_kernel<false>, grid, dim3(kSliceThreads), 0, as_stream(stream), tables,
-                     nZ, Py, Px, sites, slice_offsets, Ny, Nx, sigma, static_cast<float2*>(t_out), nullptr);
-  return check_hip(hipGetLastError(), "build_slices_kernel launch");
+  return launch_build<false>(tables, nZ, Py, Px, sites, slice_offsets, S, Ny, Nx, sigma, static_cast<float2*>(t_out),
+                             nullptr, as_stream(stream));
 }
 
 int namsa_build_potential(const float* tables, int nZ, int Py, int Px, const int* sites,
@@ -270,10 +443,8 @@ int namsa_build_potential(const float* tables, int nZ, int Py, int Px, const int
     return fail(kErrArg, "namsa_build_potential: bad arguments");
   if (S == 0) return kOk;
   if (S > 65535) return fail(kErrArg, "namsa_build_potential: S=%d exceeds the grid z limit", S);
-  dim3 grid((Nx + kTileW - 1) / kTileW, (Ny + kTileH - 1) / kTileH, S);
-  hipLaunchKernelGGL(build_slices_kernel<true>, grid, dim3(kSliceThreads), 0, as_stream(stream), tables,
-                     nZ, Py, Px, sites, slice_offsets, Ny, Nx, 0.0f, nullptr, v_out);
-  return check_hip(hipGetLastError(), "build_slices_kernel launch");
+  return launch_build<true>(tables, nZ, Py, Px, sites, slice_offsets, S, Ny, Nx, 0.0f, nullptr, v_out,
+                            as_stream(stream));
 }
 
 }  // extern "C"
