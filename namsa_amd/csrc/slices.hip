@@ -46,20 +46,24 @@ __device__ double kirkland_v(const double* p, double r) {
   return v;
 }
 
-// Mean of the os x os subsamples of table pixel i; subsample axes are
+// Subsample (dy, dx) of table pixel i; the subsample axes are
 // linspace(-range/2, range/2, os*P) (the mgrid of msa.py:141-143).
-__device__ double table_bin(const double* p, int i, int Py, int Px, int os, double range) {
+__device__ double table_sample(const double* p, int i, int dy, int dx, int Py, int Px, int os, double range) {
   const int r = i / Px, c = i % Px;
   const double half = range / 2.0;
   const double s0 = range / double(os * Py - 1), s1 = range / double(os * Px - 1);
+  const double gy = -half + double(os * r + dy) * s0;
+  const double gx = -half + double(os * c + dx) * s1;
+  return kirkland_v(p, sqrt(gy * gy + gx * gx));
+}
+
+// Mean of a pixel's os x os subsamples, sample(dy, dx).
+template <class Sample>
+__device__ double table_mean(int os, Sample sample) {
   double acc = 0.0;
   for (int dy = 0; dy < os; ++dy) {
-    const double gy = -half + double(os * r + dy) * s0;
     double row = 0.0;
-    for (int dx = 0; dx < os; ++dx) {
-      const double gx = -half + double(os * c + dx) * s1;
-      row += kirkland_v(p, sqrt(gy * gy + gx * gx));
-    }
+    for (int dx = 0; dx < os; ++dx) row += sample(dy, dx);
     acc += row / os;
   }
   return acc / os;
@@ -67,24 +71,71 @@ __device__ double table_bin(const double* p, int i, int Py, int Px, int os, doub
 
 constexpr int kTableThreads = 256;
 
-__global__ void __launch_bounds__(kTableThreads)
-atomic_tables_kernel(const double* __restrict__ params, int Py, int Px, int os, double range,
-                     float* __restrict__ tables) {
+// A table from its pixels alone, minimum first: one workgroup per element.
+__device__ void table_by_one_workgroup(const double* p, int Py, int Px, int os, double range, float* out) {
   __shared__ double red[kTableThreads / 64];
-  const double* p = params + blockIdx.x * 12;
   const int n = Py * Px;
+  const auto mean = [&](int i) {
+    return table_mean(os, [&](int dy, int dx) { return table_sample(p, i, dy, dx, Py, Px, os, range); });
+  };
   double vmin = 1.0e300;
-  for (int i = threadIdx.x; i < n; i += kTableThreads)
-    vmin = fmin(vmin, table_bin(p, i, Py, Px, os, range));
+  for (int i = threadIdx.x; i < n; i += kTableThreads) vmin = fmin(vmin, mean(i));
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) vmin = fmin(vmin, __shfl_xor(vmin, off, 64));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = vmin;
   __syncthreads();
   double m = red[0];
   for (int w = 1; w < kTableThreads / 64; ++w) m = fmin(m, red[w]);
+  for (int i = threadIdx.x; i < n; i += kTableThreads) out[i] = float(mean(i) - m);
+}
+
+// Tables shifted by the lowest of their corner pixels, which is the minimum
+// of any table that falls off outwards; table_check_kernel redoes the others.
+// Bound by the chain of FP64 instructions of one Bessel integral (about 7000
+// per subsample), so every subsample has its own thread and the workgroups
+// cover kTableThreads / os^2 pixels each; kCornerThreads more threads take
+// the corners' subsamples meanwhile, in every workgroup.  Four elements of 64
+// x 64 pixels, os = 2: 1960 us with a workgroup per element and every pixel
+// evaluated twice, 42 us now, both kernels.
+constexpr int kCornerThreads = 64;
+constexpr int kMaxSplitOs = 4;  // 4 corners of os^2 subsamples in kCornerThreads
+
+__global__ void __launch_bounds__(kTableThreads + kCornerThreads)
+atomic_tables_kernel(const double* __restrict__ params, int Py, int Px, int os, double range,
+                     float* __restrict__ tables) {
+  __shared__ double val[kTableThreads + kCornerThreads];
+  __shared__ double corner[4];
+  const double* p = params + blockIdx.y * 12;
+  const int n = Py * Px, os2 = os * os, per = kTableThreads / os2;
+  const int tid = threadIdx.x;
+  const bool edge = tid >= kTableThreads;
+  const int slot = (edge ? tid - kTableThreads : tid) / os2, sub = (edge ? tid - kTableThreads : tid) % os2;
+  const auto corner_pixel = [&](int k) { return (k >> 1) * (Py - 1) * Px + (k & 1) * (Px - 1); };
+  const int i = edge ? (slot < 4 ? corner_pixel(slot) : n) : static_cast<int>(blockIdx.x) * per + slot;
+  if (i < n && (edge || slot < per)) val[tid] = table_sample(p, i, sub / os, sub % os, Py, Px, os, range);
+  __syncthreads();
+  const int first = edge ? kTableThreads + slot * os2 : slot * os2;
+  const bool lead = sub == 0 && i < n && (edge || slot < per);
+  double mean = 0.0;
+  if (lead) mean = table_mean(os, [&](int dy, int dx) { return val[first + dy * os + dx]; });
+  if (lead && edge) corner[slot] = mean;
+  __syncthreads();
+  if (lead && !edge)
+    tables[static_cast<long long>(blockIdx.y) * n + i] =
+        float(mean - fmin(fmin(corner[0], corner[1]), fmin(corner[2], corner[3])));
+}
+
+// A table with a value below its corners' (or a NaN) is made again from its
+// own minimum.
+__global__ void __launch_bounds__(kTableThreads)
+table_check_kernel(const double* __restrict__ params, int Py, int Px, int os, double range, int force,
+                   float* __restrict__ tables) {
+  const int n = Py * Px;
   float* out = tables + static_cast<long long>(blockIdx.x) * n;
-  for (int i = threadIdx.x; i < n; i += kTableThreads)
-    out[i] = float(table_bin(p, i, Py, Px, os, range) - m);
+  int bad = force;
+  if (!force)
+    for (int i = threadIdx.x; i < n; i += kTableThreads) bad |= !(out[i] >= 0.0f);
+  if (__syncthreads_or(bad)) table_by_one_workgroup(params + blockIdx.x * 12, Py, Px, os, range, out);
 }
 
 // ------------------------------------------------------------------ slice builder
@@ -419,8 +470,17 @@ int namsa_atomic_tables(const double* params, int nZ, int Py, int Px, double ran
       oversample * static_cast<long long>(Py) < 2 || oversample * static_cast<long long>(Px) < 2)
     return fail(kErrArg, "namsa_atomic_tables: bad arguments (nZ=%d Py=%d Px=%d os=%d)", nZ, Py,
                 Px, oversample);
-  hipLaunchKernelGGL(atomic_tables_kernel, dim3(nZ), dim3(kTableThreads), 0, as_stream(stream),
-                     params, Py, Px, oversample, range, tables);
+  hipStream_t st = as_stream(stream);
+  // one thread per subsample while the corners' fit their wavefront (os <= 4)
+  const bool split = oversample <= kMaxSplitOs && nZ <= 65535;
+  if (split) {
+    const int per = kTableThreads / (oversample * oversample);
+    const long long n = static_cast<long long>(Py) * Px;
+    hipLaunchKernelGGL(atomic_tables_kernel, dim3(static_cast<unsigned>((n + per - 1) / per), nZ),
+                       dim3(kTableThreads + kCornerThreads), 0, st, params, Py, Px, oversample, range, tables);
+  }
+  hipLaunchKernelGGL(table_check_kernel, dim3(nZ), dim3(kTableThreads), 0, st, params, Py, Px, oversample, range,
+                     split ? 0 : 1, tables);
   return check_hip(hipGetLastError(), "atomic_tables_kernel launch");
 }
 
