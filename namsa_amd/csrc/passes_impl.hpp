@@ -95,6 +95,7 @@ struct ColS {
   static constexpr int N = N_, E = E_, C = C_, W = W_, K = K_;
   using RL = RL_;
   static constexpr bool PF = PF_, NT = NT_, DB = DB_, CT = CT_, PG = PG_, SB = SB_, LR = LR_;
+  using F = Fft<N, E, RL, CT, LR>;
   static constexpr int threads() { return C * (N / E); }
 };
 
@@ -311,7 +312,7 @@ __global__ void __launch_bounds__(kRowThreads, S::W > 0 ? S::W : 1) row_step_tr_
 template <class S, int OP>
 __global__ void __launch_bounds__(S::threads(), S::W > 0 ? S::W : 1) col_kernel(ColArgs a) {
   constexpr int N = S::N, E = S::E, C = S::C;
-  using F = Fft<N, E, typename S::RL, S::CT, S::LR>;
+  using F = typename S::F;
   constexpr int T = F::T;
   constexpr int NW = S::threads() / 64;
   constexpr bool LOADS = OP != COL_PROBE;
@@ -561,8 +562,16 @@ int launch_col_op(ColArgs& a, hipStream_t st) {
   if constexpr (S::W > 0) {
     // Schedules sized for several workgroups per CU: one (strip, image) task
     // per workgroup, which the dispatcher deals out to the CU slots as they
-    // free up, so the strips x images tasks balance whatever their count.
-    const long long grid = static_cast<long long>(a.n_strips) * ((a.B + S::K - 1) / S::K);
+    // free up, so the strips x images tasks balance whatever their count.  A
+    // workgroup takes up to K images of its strip: the most that leave 4/3 as
+    // many workgroups as are resident at one time (1024^2, K = 4, slice step:
+    // 4 images 56 us with one workgroup per strip, 36 with one per task; 8
+    // images 67 and 52; 32 images 162 with 4 each, 167 with one).  The images
+    // do not interact, so the split does not change a result.
+    const auto groups = [&](int k) { return (a.B + k - 1) / k; };
+    int k_img = S::K;
+    while (k_img > 1 && 3LL * a.n_strips * groups(k_img) < 4LL * cap) --k_img;
+    const long long grid = static_cast<long long>(a.n_strips) * groups(k_img);
     if (grid > 0x7fffffffLL) return fail(kErrArg, "column pass: %lld tasks in one launch", grid);
     hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(grid)), dim3(S::threads()), 0, st, a);
     return check_hip(hipGetLastError(), "column pass launch");
@@ -620,8 +629,21 @@ int launch_row(int op, const RowArgs& a, hipStream_t st) {
   }
 }
 
-template <class S, class Base>
+// Narrow: the same transform in narrower strips, which PROP launches of few
+// strips and images take: while its (strip, image) tasks fit one workgroup
+// per CU, twice the workgroups with half the lines to wait for are faster
+// (slice step of one image: 192^2 10.3 -> 9.4 us, 256^2 9.4 -> 8.2, 512^2 10.8
+// -> 9.6, 1024^2 20.1 -> 17.5; at two tasks per CU the two are equal or the
+// wide one is ahead).  Same operations per column: the bits do not depend on
+// it, as long as both read the propagator the same way (PG).
+template <class S, class Base, class Narrow = void>
 int launch_col(int op, ColArgs& a, hipStream_t st) {
+  if constexpr (!std::is_void<Narrow>::value) {
+    static_assert(Narrow::C < S::C && Narrow::PG == S::PG && std::is_same<typename Narrow::F, typename S::F>::value,
+                  "a narrow form only changes the strip");
+    const long long strips = (a.band_hi + Narrow::C - 1) / Narrow::C - a.band_lo / Narrow::C;
+    if (op == COL_PROP && strips * a.B <= device_cu_count()) return launch_col_op<Narrow, COL_PROP>(a, st);
+  }
   if (op == COL_PROP) return launch_col_op<S, COL_PROP>(a, st);
   // the multi-workgroup schedules' readout (one task per (strip, image),
   // detector reductions per task) is 20-50% slower than the base schedule's

@@ -3,7 +3,8 @@
 // Names read: e<E> = elements per thread, r<radices>, c<C> = column tile,
 // pf = next row/tile prefetched, nt = non-temporal wave traffic, ct = compact
 // twiddles (one register pair per butterfly, higher powers formed in the stage),
-// w<k> = register budget for at least k wavefronts per SIMD.
+// w<k> = register budget for at least k wavefronts per SIMD, i<k> = up to k
+// images per workgroup.  Types ending in N are the narrow forms of launch_col.
 #include "passes_impl.hpp"
 
 #ifndef NAMSA_PASS_N
@@ -19,12 +20,13 @@ using C0 = ColS<128, 8, Radices<8, 4, 4>, 16, false, false>;
 using C1 = ColS<128, 8, Radices<8, 4, 4>, 8, true, false>;
 using C2 = ColS<128, 8, Radices<8, 4, 4>, 16, false, false, false, false, 4, true, true>;
 using R2 = RowS<128, 8, Radices<8, 4, 4>, false, false, false, 6>;
+using C2N = ColS<128, 8, Radices<8, 4, 4>, 8, false, false, false, false, 5, true, true>;
 static const RowSchedEntry kRows[] = {{"e8.r844", launch_row<R0, R0>},
                                       {"e8.r844.pf", launch_row<R1, R0>},
                                       {"e8.r844.w6", launch_row<R2, R0>}};
 static const ColSchedEntry kCols[] = {{"e8.r844.c16", launch_col<C0, C0>, 16},
                                       {"e8.r844.c8.pf", launch_col<C1, C0>, 8},
-                                      {"e8.r844.c16.pg.sb.w4", launch_col<C2, C0>, 16}};
+                                      {"e8.r844.c16.pg.sb.w4", launch_col<C2, C0, C2N>, 16}};
 #elif NAMSA_PASS_N == 192
 using R0 = RowS<192, 12, Radices<3, 4, 4, 4>, false, false>;
 using R1 = RowS<192, 12, Radices<3, 4, 4, 4>, true, false>;
@@ -34,6 +36,8 @@ using R2 = RowS<192, 12, Radices<12, 4, 4>, false, false>;
 using R3 = RowS<192, 12, Radices<12, 4, 4>, true, false>;
 using C2 = ColS<192, 12, Radices<12, 4, 4>, 16, false, false>;
 using C3 = ColS<192, 12, Radices<12, 4, 4>, 8, true, false>;
+using C4 = ColS<192, 12, Radices<12, 4, 4>, 16, false, false, false, false, 4, false, true, 2>;
+using C4N = ColS<192, 12, Radices<12, 4, 4>, 8, false, false, false, false, 0, false, true>;
 static const RowSchedEntry kRows[] = {{"e12.r3444", launch_row<R0, R0>},
                                       {"e12.r3444.pf", launch_row<R1, R0>},
                                       {"e12.r12.4.4", launch_row<R2, R0>},
@@ -41,7 +45,8 @@ static const RowSchedEntry kRows[] = {{"e12.r3444", launch_row<R0, R0>},
 static const ColSchedEntry kCols[] = {{"e12.r3444.c16", launch_col<C0, C0>, 16},
                                       {"e12.r3444.c8.pf", launch_col<C1, C0>, 8},
                                       {"e12.r12.4.4.c16", launch_col<C2, C0>, 16},
-                                      {"e12.r12.4.4.c8.pf", launch_col<C3, C0>, 8}};
+                                      {"e12.r12.4.4.c8.pf", launch_col<C3, C0>, 8},
+                                      {"e12.r12.4.4.c16.sb.w4.i2", launch_col<C4, C0, C4N>, 16}};
 #elif NAMSA_PASS_N == 256
 using R0 = RowS<256, 8, Radices<8, 8, 4>, false, false>;
 using R1 = RowS<256, 8, Radices<8, 8, 4>, true, false>;
@@ -50,13 +55,16 @@ using R3 = RowS<256, 8, Radices<8, 8, 4>, false, false, false, 5>;
 using C0 = ColS<256, 8, Radices<8, 8, 4>, 16, false, false>;
 using C1 = ColS<256, 8, Radices<8, 8, 4>, 8, true, false>;
 using C2 = ColS<256, 16, Radices<16, 16>, 16, true, false>;
+using C3 = ColS<256, 8, Radices<8, 8, 4>, 8, false, false, false, false, 6, false, true, 2>;
+using C3N = ColS<256, 8, Radices<8, 8, 4>, 4, false, false, false, false, 0, false, true>;
 static const RowSchedEntry kRows[] = {{"e8.r884", launch_row<R0, R0>},
                                       {"e8.r884.pf", launch_row<R1, R0>},
                                       {"e16.r16.16.pf", launch_row<R2, R0>},
                                       {"e8.r884.w5", launch_row<R3, R0>}};
 static const ColSchedEntry kCols[] = {{"e8.r884.c16", launch_col<C0, C0>, 16},
                                       {"e8.r884.c8.pf", launch_col<C1, C0>, 8},
-                                      {"e16.r16.16.c16.pf", launch_col<C2, C0>, 16}};
+                                      {"e16.r16.16.c16.pf", launch_col<C2, C0>, 16},
+                                      {"e8.r884.c8.sb.w6.i2", launch_col<C3, C0, C3N>, 8}};
 #elif NAMSA_PASS_N == 384
 using R0 = RowS<384, 12, Radices<3, 2, 4, 4, 4>, false, false>;
 using R1 = RowS<384, 12, Radices<3, 2, 4, 4, 4>, true, false>;
@@ -116,6 +124,8 @@ using C14 = ColS<512, 8, Radices<8, 8, 8>, 16, true, false, true, true>;
 using C15 = ColS<512, 8, Radices<8, 8, 8>, 8, false, false, false, true, 6, true, true>;
 using C16 = ColS<512, 8, Radices<8, 8, 8>, 8, false, false, false, false, 6, true, true>;
 using C17 = ColS<512, 8, Radices<8, 8, 8>, 8, false, false, false, false, 6, true, true, 1, true>;
+using C15N = ColS<512, 8, Radices<8, 8, 8>, 4, false, false, false, true, 6, true, true>;
+using C17N = ColS<512, 8, Radices<8, 8, 8>, 4, false, false, false, false, 6, true, true, 1, true>;
 using R5 = RowS<512, 8, Radices<8, 8, 8>, false, false, true>;
 using R6 = RowS<512, 8, Radices<8, 8, 8>, false, false, false, 5>;
 static const RowSchedEntry kRows[] = {{"e8.r888", launch_row<R0, R0>},
@@ -140,9 +150,9 @@ static const ColSchedEntry kCols[] = {{"e16.r888.c16", launch_col<C0, C0>, 16},
                                       {"e16.r16.16.2.c16.pf", launch_col<C12, C0>, 16},
                                       {"e8.r888.c16.pf.ct", launch_col<C13, C0>, 16},
                                       {"e8.r888.c16.db.pf.ct", launch_col<C14, C0>, 16},
-                                      {"e8.r888.c8.pg.sb.w6.ct", launch_col<C15, C0>, 8, "e8.r888.c8.lr.pg.sb.w6"},
+                                      {"e8.r888.c8.pg.sb.w6.ct", launch_col<C15, C0, C15N>, 8, "e8.r888.c8.lr.pg.sb.w6"},
                                       {"e8.r888.c8.pg.sb.w6", launch_col<C16, C0>, 8},
-                                      {"e8.r888.c8.lr.pg.sb.w6", launch_col<C17, C0>, 8}};
+                                      {"e8.r888.c8.lr.pg.sb.w6", launch_col<C17, C0, C17N>, 8}};
 #elif NAMSA_PASS_N == 768
 using R0 = RowS<768, 12, Radices<3, 4, 4, 4, 4>, false, false>;
 using R1 = RowS<768, 12, Radices<3, 4, 4, 4, 4>, true, false>;
@@ -160,6 +170,8 @@ using C7 = ColS<768, 12, Radices<12, 4, 4, 4>, 8, false, false, false, true, 4, 
 using C8 = ColS<768, 12, Radices<12, 4, 4, 4>, 8, true, false, true>;
 using C9 = ColS<768, 12, Radices<12, 4, 4, 4>, 8, false, false, false, true, 4, true, true>;
 using C10 = ColS<768, 12, Radices<12, 4, 4, 4>, 8, false, false, false, false, 4, true, true>;
+using C9N = ColS<768, 12, Radices<12, 4, 4, 4>, 4, false, false, false, true, 4, true, true>;
+using C10N = ColS<768, 12, Radices<12, 4, 4, 4>, 4, false, false, false, false, 4, true, true>;
 static const RowSchedEntry kRows[] = {{"e12.r34444", launch_row<R0, R0>},
                                       {"e12.r34444.pf", launch_row<R1, R0>},
                                       {"e12.r34444.ct", launch_row<R2, R0>},
@@ -174,8 +186,8 @@ static const ColSchedEntry kCols[] = {{"e12.r34444.c8", launch_col<C0, C0>, 8},
                                       {"e12.r34444.c8.sb.w4.i2.ct", launch_col<C6, C0>, 8, "e12.r34444.c8.db.pf"},
                                       {"e12.r12.4.4.4.c8.sb.w4.i2.ct", launch_col<C7, C0>, 8, "e12.r12.4.4.4.c8.db.pf"},
                                       {"e12.r12.4.4.4.c8.db.pf", launch_col<C8, C0>, 8},
-                                      {"e12.r12.4.4.4.c8.pg.sb.w4.ct", launch_col<C9, C0>, 8},
-                                      {"e12.r12.4.4.4.c8.pg.sb.w4", launch_col<C10, C0>, 8}};
+                                      {"e12.r12.4.4.4.c8.pg.sb.w4.ct", launch_col<C9, C0, C9N>, 8},
+                                      {"e12.r12.4.4.4.c8.pg.sb.w4", launch_col<C10, C0, C10N>, 8}};
 #elif NAMSA_PASS_N == 1024
 using R0 = RowS<1024, 16, Radices<16, 8, 8>, false, false>;
 using R1 = RowS<1024, 16, Radices<16, 8, 8>, true, false>;
@@ -197,14 +209,16 @@ using C4 = ColS<1024, 16, Radices<16, 8, 8>, 8, false, false, false, false, 4, t
 using C5 = ColS<1024, 16, Radices<16, 8, 8>, 8, false, false, false, true, 4, true, true>;
 using C6 = ColS<1024, 16, Radices<16, 8, 8>, 8, false, false, false, true, 4, false, true, 4>;
 using C7 = ColS<1024, 16, Radices<16, 8, 8>, 8, false, false, false, false, 4, true, true, 1, true>;
+using C6N = ColS<1024, 16, Radices<16, 8, 8>, 4, false, false, false, true, 0, false, true>;
+using C7N = ColS<1024, 16, Radices<16, 8, 8>, 4, false, false, false, false, 4, true, true, 1, true>;
 static const ColSchedEntry kCols[] = {{"e16.r16.8.8.c8", launch_col<C0, C0>, 8},
                                       {"e16.r16.8.8.c8.pf", launch_col<C1, C0>, 8},
                                       {"e8.r8844.c8", launch_col<C2, C0>, 8},
                                       {"e16.r16.8.8.c8.pf.ct", launch_col<C3, C0>, 8},
                                       {"e16.r16.8.8.c8.pg.sb.w4", launch_col<C4, C0>, 8},
                                       {"e16.r16.8.8.c8.pg.sb.w4.ct", launch_col<C5, C0>, 8},
-                                      {"e16.r16.8.8.c8.sb.w4.i4.ct", launch_col<C6, C0>, 8, "e16.r16.8.8.c8.lr.pg.sb.w4"},
-                                      {"e16.r16.8.8.c8.lr.pg.sb.w4", launch_col<C7, C0>, 8}};
+                                      {"e16.r16.8.8.c8.sb.w4.i4.ct", launch_col<C6, C0, C6N>, 8, "e16.r16.8.8.c8.lr.pg.sb.w4"},
+                                      {"e16.r16.8.8.c8.lr.pg.sb.w4", launch_col<C7, C0, C7N>, 8}};
 #elif NAMSA_PASS_N == 2048
 using R0 = RowS<2048, 16, Radices<16, 16, 8>, false, false>;
 using R1 = RowS<2048, 16, Radices<16, 16, 8>, true, false>;
