@@ -15,14 +15,16 @@
 // strides and the base pointer allow it, and the next K tile is loaded into
 // registers while the matrix cores work on the current one.  MFMA operands
 // come out of LDS as 16-byte reads.  With split_k > 1 the K range is divided
-// over blockIdx.z and partial products are added to C with FP32 atomics (C
-// must then already hold beta*C).
+// over workgroups and partial products are added to C with FP32 atomics (C
+// must then already hold beta*C); gemm_split_kernel takes the small products
+// over a long contiguous K.
 //
 // MFMA 32x32x16 operand layout (lane l, 8 bf16 per operand register set):
 //   A: row l%32, k = 8*(l/32) + e      B: column l%32, k = 8*(l/32) + e
 //   D: 16 floats, register r holds row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "common.hpp"
@@ -265,6 +267,109 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(GemmArgs g) {
   store_block(g, b, acc, 0, lane);
 }
 
+// Eight consecutive k of one operand row as an MFMA register set, rounded to
+// bf16; `left` of them exist, the others are 0.  Rows need not be 16-byte
+// aligned: the loads only assume 4-byte alignment.
+struct alignas(4) F4 {
+  float v[4];
+};
+
+__device__ __forceinline__ bf16x8 load_k8(const float* __restrict__ p, int left) {
+  bf16x8 h;
+  if (left >= 8) {
+    const F4 a = *reinterpret_cast<const F4*>(p), b = *reinterpret_cast<const F4*>(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      h[e] = __bf16(a.v[e]);
+      h[e + 4] = __bf16(b.v[e]);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) h[e] = __bf16(e < left ? p[e] : 0.0f);
+  }
+  return h;
+}
+
+// Split-K products of few rows and columns (M <= 32 MT, N <= 32 NT) over a
+// long K with both operands contiguous along it: the weight gradients, sums
+// over every pixel of a batch.  Bound by reading the operands once, so a
+// workgroup's four wavefronts each take every fourth step of 32 k of its K
+// range, with all 32 x 32 blocks of the result in their accumulators and the
+// operands read straight into the MFMA layout (a tile staged through LDS left
+// three of four wavefronts without a block and one load in flight per
+// barrier).  The wavefronts' blocks are summed through LDS and added to C with
+// one FP32 atomic per value and workgroup, so one workgroup per CU: two per CU
+// were no faster.  Over 462,400 k: 32 x 32 175 -> 30 us (3.9 TB/s), 64 x 32 239
+// -> 42, 32 sums 185 -> 22, against 112 staged workgroups.
+template <int MT, int NT>
+__global__ void __launch_bounds__(256) gemm_split_kernel(GemmArgs g, int k_per) {
+  __shared__ float part[4][MT * NT][16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long long b = blockIdx.y;
+  const int row = lane & 31, kh = 8 * (lane >> 5);
+  const int k_begin = blockIdx.x * k_per, k_end = min(g.K, k_begin + k_per);
+  // lanes past the last row or column read that row: what they add to goes
+  // into values that are not stored
+  const float* A[MT];
+  const float* B[NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) A[i] = g.A + b * g.sAb + min(32 * i + row, g.M - 1) * g.sAi + kh;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) B[j] = g.B + b * g.sBb + min(32 * j + row, g.N - 1) * g.sBj + kh;
+  f32x16 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+#pragma unroll 2
+  for (int k0 = k_begin + 32 * wave; k0 < k_end; k0 += 128) {
+    bf16x8 a[MT][2], c[NT][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int left = k_end - k0 - kh - 16 * h;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) a[i][h] = load_k8(A[i] + k0 + 16 * h, left);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) c[j][h] = load_k8(B[j] + k0 + 16 * h, left);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][h], c[j][h], acc[i][j], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < MT * NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave][t][r][lane] = acc[t / NT][t % NT][r];
+  __syncthreads();
+  // values in row-major order over the threads, so that one atomic
+  // instruction covers neighbouring addresses (a column of sums, N = 1, took
+  // 48 us with a wavefront's registers stored one by one, 32 lines' worth of
+  // atomics on one line)
+  float* C = g.C + b * g.sCb;
+  for (int v = threadIdx.x; v < g.M * g.N; v += 256) {
+    const int i = v / g.N, j = v % g.N;
+    const int t = (i >> 5) * NT + (j >> 5), r = 4 * ((i & 31) >> 3) + (i & 3), l = (j & 31) + 32 * ((i >> 2) & 1);
+    const float sum = (part[0][t][r][l] + part[1][t][r][l]) + (part[2][t][r][l] + part[3][t][r][l]);
+    atomicAdd(C + i * g.sCi + j * g.sCj, g.alpha * sum);
+  }
+}
+
+template <int MT, int NT>
+int launch_split(const GemmArgs& g, hipStream_t st) {
+  // one workgroup per CU, each at least one step of 32 k per wavefront
+  const int cus = device_cu_count();
+  const int groups = std::max(1, std::min((g.K + 127) / 128, (cus + g.batch - 1) / g.batch));
+  const int k_per = ((g.K + groups - 1) / groups + 127) / 128 * 128;
+  hipLaunchKernelGGL((gemm_split_kernel<MT, NT>), dim3((g.K + k_per - 1) / k_per, g.batch), dim3(256), 0, st, g, k_per);
+  return check_hip(hipGetLastError(), "gemm_split_kernel launch");
+}
+
 template <int WM, int WN>
 int launch_gemm(const GemmArgs& g, hipStream_t st) {
   constexpr int TM = 32 * WM, TN = 32 * WN;
@@ -300,6 +405,10 @@ int namsa_gemm_bf16(const float* A, long long sAb, long long sAi, long long sAk,
   if (M <= 32 && N <= 32 && split_k == 1 && batch >= 64) {
     hipLaunchKernelGGL(gemm_small_kernel, dim3(static_cast<unsigned>(batch)), dim3(256), 0, st, g);
     return check_hip(hipGetLastError(), "gemm_small_kernel launch");
+  }
+  if (split_k > 1 && sAk == 1 && sBk == 1 && M <= 64 && N <= 64) {
+    if (M <= 32) return N <= 32 ? launch_split<1, 1>(g, st) : launch_split<1, 2>(g, st);
+    return N <= 32 ? launch_split<2, 1>(g, st) : launch_split<2, 2>(g, st);
   }
   if (N <= 32) return launch_gemm<4, 1>(g, st);
   if (M <= 32) return launch_gemm<1, 4>(g, st);

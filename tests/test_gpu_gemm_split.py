@@ -1,0 +1,43 @@
+"""Split-K products with both operands contiguous along K (the corrector's
+weight gradients): every combination of one and two 32-wide blocks with ragged
+edges, K on both sides of a wavefront's step and a workgroup's share, rows and
+pointers off 16 bytes, a zero-stride operand, batches and a strided C.  Against
+float64 products of the bf16-rounded operands: FP32 accumulation, 2e-5 of the
+norm of |A| |B|."""
+import numpy as np
+import pytest
+
+import namsa_amd._lib as L
+from tests.test_gpu_corrector_kernels import bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K,batch,pad,off,zero", [
+    (1, 1, 1, 1, 0, 0, False), (32, 32, 31, 1, 1, 1, False), (32, 32, 33, 2, 3, 2, False), (2, 64, 127, 1, 0, 0, False),
+    (64, 1, 1000, 1, 0, 0, True), (33, 47, 129, 3, 2, 1, False), (64, 64, 4099, 1, 1, 3, False),
+    (7, 32, 70001, 1, 0, 0, False), (32, 1, 40000, 2, 1, 0, True), (64, 33, 33000, 1, 0, 0, False)])
+def test_split_products(gpu, M, N, K, batch, pad, off, zero):
+    import torch
+
+    print(f"split gemm M={M} N={N} K={K} batch={batch} pad={pad} off={off} zero stride={zero}", flush=True)
+    rng = np.random.default_rng(K + M)
+    sA, sB = K + pad, 0 if zero else K + pad
+    A = rng.standard_normal(off + batch * M * sA + K).astype(np.float32)
+    B = rng.standard_normal(off + batch * max(1, N * sB) + K).astype(np.float32)
+    bA, bB = M * sA, N * sB
+    sC = (1, M + 2)                                   # C stored column by column, padded
+    C0 = rng.standard_normal(batch * N * (M + 2)).astype(np.float32)
+    Ad, Bd, Cd = (torch.from_numpy(x).to(gpu) for x in (A, B, C0.copy()))
+    L.call("namsa_gemm_bf16", L.ptr(Ad[off:]), bA, sA, 1, L.ptr(Bd[off:]), bB, 1, sB, L.ptr(Cd), N * (M + 2), *sC, M, N,
+           K, batch, 3, np.float32(0.5), np.float32(0.0), None, 0, 0, None, L.stream_handle())
+    got = Cd.cpu().numpy().astype(np.float64)
+    touched = np.zeros(got.shape, bool)
+    for b in range(batch):
+        a = bf16(np.stack([A[off + b * bA + i * sA:][:K] for i in range(M)]))
+        w = bf16(np.stack([B[off + b * bB + j * sB:][:K] for j in range(N)]))
+        at = b * N * (M + 2) + np.arange(M)[:, None] * sC[0] + np.arange(N)[None, :] * sC[1]
+        touched[at] = True
+        err = np.linalg.norm(got[at] - C0[at] - 0.5 * (a @ w.T)) / np.linalg.norm(np.abs(a) @ np.abs(w).T)
+        assert err < 2e-5, (b, err)
+    assert np.array_equal(got[~touched], C0[~touched])
