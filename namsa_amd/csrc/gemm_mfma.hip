@@ -11,10 +11,11 @@
 // takes 32 x 128 tiles and the rest 64 x 64 -- no wavefront idles on a
 // 32-wide side -- and batches of many items that each fit one 32 x 32 block
 // take one wavefront per item.  Operand tiles of K = 32 are staged through LDS as bf16 with
-// k contiguous: the unit-stride axis is read with 16-byte loads where the
-// strides and the base pointer allow it, and the next K tile is loaded into
+// k contiguous: the unit-stride axis is read with 16-byte loads (at any 4-byte
+// aligned address), and the next K tile is loaded into
 // registers while the matrix cores work on the current one.  MFMA operands
-// come out of LDS as 16-byte reads.  With split_k > 1 the K range is divided
+// come out of LDS as 16-byte reads.  Pointwise layers over many columns run without
+// LDS (gemm_pointwise_kernel).  With split_k > 1 the K range is divided
 // over workgroups and partial products are added to C with FP32 atomics (C
 // must then already hold beta*C); gemm_split_kernel takes the small products
 // over a long contiguous K.
@@ -59,6 +60,11 @@ __device__ __forceinline__ float gelu_tanh(float x) {
   return 0.5f * x * (1.0f + tanhf(c * (x + 0.044715f * x * x * x)));
 }
 
+// Four consecutive floats at any 4-byte aligned address, one 16-byte load.
+struct alignas(4) F4 {
+  float v[4];
+};
+
 // One operand tile of R rows (i for A, j for B) by kTK k values, element
 // (r, k) at base + (r0 + r) * sr + (k0 + k) * sk, valid for r0 + r < rows
 // and k0 + k < k_end.  Each thread carries G groups of 4 elements that are
@@ -83,11 +89,9 @@ struct Tile {
       }
       const int gr = r0 + r, gk = k0 + k;
       if (vec && (kfast ? (gr < rows && gk + 3 < k_end) : (gr + 3 < rows && gk < k_end))) {
-        const float4 f = *reinterpret_cast<const float4*>(base + gr * sr + gk * sk);
-        v[q][0] = f.x;
-        v[q][1] = f.y;
-        v[q][2] = f.z;
-        v[q][3] = f.w;
+        const F4 f = *reinterpret_cast<const F4*>(base + gr * sr + gk * sk);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[q][e] = f.v[e];
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -117,14 +121,6 @@ struct Tile {
   }
 };
 
-// 16-byte loads along the unit-stride axis need that stride to be 1, the
-// other stride and the batch stride to keep 4-float alignment, and an
-// aligned base.
-__device__ __forceinline__ bool vec_ok(const float* base, long long s_unit, long long s_other, long long s_batch) {
-  return s_unit == 1 && (s_other & 3) == 0 && (s_batch & 3) == 0 &&
-         (reinterpret_cast<uintptr_t>(base) & 15) == 0;
-}
-
 template <int WM, int WN>
 __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g) {
   constexpr int TM = 32 * WM, TN = 32 * WN;
@@ -148,8 +144,8 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g) {
   // A rows are i (stride sAi), B rows are j (stride sBj); k is the column
   const bool a_kfast = g.sAk == 1 || (g.sAi != 1 && g.sAk <= g.sAi);
   const bool b_kfast = g.sBk == 1 || (g.sBj != 1 && g.sBk <= g.sBj);
-  const bool a_vec = a_kfast ? vec_ok(g.A, g.sAk, g.sAi, g.sAb) : vec_ok(g.A, g.sAi, g.sAk, g.sAb);
-  const bool b_vec = b_kfast ? vec_ok(g.B, g.sBk, g.sBj, g.sBb) : vec_ok(g.B, g.sBj, g.sBk, g.sBb);
+  const bool a_vec = (a_kfast ? g.sAk : g.sAi) == 1;
+  const bool b_vec = (b_kfast ? g.sBk : g.sBj) == 1;
 
   f32x16 acc;
 #pragma unroll
@@ -204,14 +200,16 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g) {
   }
 }
 
-// Epilogue of one 32 x 32 MFMA block of item b, rows i0 .. i0 + 31:
+// Epilogue of one 32 x 32 MFMA block of item b, rows i0 .. i0 + 31 and columns
+// j0 .. j0 + 31:
 // C = alpha acc + beta C (+ bias), optionally keeping the pre-activation in P
 // and applying GELU.  Register r of lane l holds row 8(r/4) + 4(l/32) + r%4,
 // column l%32.
-__device__ __forceinline__ void store_block(const GemmArgs& g, long long b, const f32x16& acc, int i0, int lane) {
+__device__ __forceinline__ void store_block(const GemmArgs& g, long long b, const f32x16& acc, int i0, int j0,
+                                            int lane) {
   float* C = g.C + b * g.sCb;
   float* P = g.P ? g.P + b * g.sCb : nullptr;
-  const int j = lane & 31;
+  const int j = j0 + (lane & 31);
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int i = i0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
@@ -264,16 +262,12 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(GemmArgs g) {
   if (wave > 0) return;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] += part[0][r][lane] + part[1][r][lane] + part[2][r][lane];
-  store_block(g, b, acc, 0, lane);
+  store_block(g, b, acc, 0, 0, lane);
 }
 
 // Eight consecutive k of one operand row as an MFMA register set, rounded to
 // bf16; `left` of them exist, the others are 0.  Rows need not be 16-byte
 // aligned: the loads only assume 4-byte alignment.
-struct alignas(4) F4 {
-  float v[4];
-};
-
 __device__ __forceinline__ bf16x8 load_k8(const float* __restrict__ p, int left) {
   bf16x8 h;
   if (left >= 8) {
@@ -360,6 +354,109 @@ __global__ void __launch_bounds__(256) gemm_split_kernel(GemmArgs g, int k_per) 
   }
 }
 
+// Pointwise layers: few rows and a short K (M <= 32 MT, K <= 16 KS) over a
+// long unit-stride N, the pixels of a batch.  Bound by streaming B and C once
+// (a tile staged through LDS wrote its bf16 operands two bytes at a time and
+// had nothing in flight across its barriers).  A wavefront holds A in the MFMA
+// layout and takes PB blocks of 32 columns, every read of B issued before the
+// first product.  Reads and writes are buffer accesses: a scalar row offset
+// and one lane offset (with pointers the 64-bit addresses took 250 registers),
+// rows past K read 0 and rows past M are not written, being past the buffer's
+// end (the launcher checks sBk, sCi >= N and 31-bit sizes).  The products run
+// over k in the order of the staged kernel.  Over 462,400 columns: 32
+// x 32 with bias 47 -> 32 us, with beta 57 -> 31, 32 x 7 44 -> 16, 64 x 32 with
+// GELU 109 -> 82 (296 MB).
+constexpr int kRawBuffer = 0x00020000;  // gfx9 raw-buffer resource word 3
+
+template <int MT, int KS, int PB, bool BIAS>
+__global__ void __launch_bounds__(256) gemm_pointwise_kernel(GemmArgs g) {
+  const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
+  const int sB = static_cast<int>(g.sBk) * 4, sC = static_cast<int>(g.sCi) * 4;  // row pitches in bytes
+  const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(g.B), 0, (g.K - 1) * sB + g.N * 4, kRawBuffer);
+  const auto rc = __builtin_amdgcn_make_buffer_rsrc(g.C, 0, (g.M - 1) * sC + g.N * 4, kRawBuffer);
+  const auto rp = __builtin_amdgcn_make_buffer_rsrc(g.P, 0, g.P ? (g.M - 1) * sC + g.N * 4 : 0, kRawBuffer);
+  const int j0 = 32 * PB * (blockIdx.x * 4 + (threadIdx.x >> 6)) + col;
+  float x[PB][KS][8];
+#pragma unroll
+  for (int p = 0; p < PB; ++p)
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        x[p][s][e] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(rb, 8 * half * sB + 4 * (j0 + 32 * p), (16 * s + e) * sB, 0));
+  bf16x8 a[MT][KS];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int row = 32 * i + col, k = 16 * s + 8 * half + e;
+        const float w = g.A[min(row, g.M - 1) * g.sAi + min(k, g.K - 1) * g.sAk];
+        a[i][s][e] = __bf16(row < g.M && k < g.K ? w : 0.0f);
+      }
+  float bias[BIAS ? MT : 1][16];  // read here: a read after the products would wait for all of x
+  if constexpr (BIAS) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bias[i][r] = g.bias[min(32 * i + 8 * (r >> 2) + 4 * half + (r & 3), g.M - 1)];
+  }
+#pragma unroll
+  for (int p = 0; p < PB; ++p) {
+    const int j = j0 + 32 * p;
+    bf16x8 b[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) b[s][e] = __bf16(x[p][s][e]);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      f32x16 acc;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][s], b[s], acc, 0, 0, 0);
+      if (j >= g.N) continue;
+      const int at = 4 * half * sC + 4 * j;
+      float old[16];
+      if (g.beta != 0.0f) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          old[r] = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(rc, at, (32 * i + 8 * (r >> 2) + (r & 3)) * sC, 0));
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row0 = 32 * i + 8 * (r >> 2) + (r & 3);
+        float v = g.alpha * acc[r];
+        if (g.beta != 0.0f) v += g.beta * old[r];
+        if constexpr (BIAS) v += bias[i][r];
+        if (g.bias_mode == 2) v += g.bias[j];
+        if (g.gelu) {
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rp, at, row0 * sC, 0);
+          v = gelu_tanh(v);
+        }
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rc, at, row0 * sC, 0);
+      }
+    }
+  }
+}
+
+template <int MT, int KS>
+int launch_pointwise(const GemmArgs& g, hipStream_t st) {
+  // blocks per wavefront: 4 with a bias (its 16 reads per 32 rows are then
+  // paid once per 128 columns) and for K = 32, else 2
+  constexpr int PB = KS == 2 ? 4 : 2;
+  const auto grid = [&](int pb) { return dim3((g.N + 128 * pb - 1) / (128 * pb)); };
+  if (g.bias_mode == 1)
+    hipLaunchKernelGGL((gemm_pointwise_kernel<MT, KS, 4, true>), grid(4), dim3(256), 0, st, g);
+  else
+    hipLaunchKernelGGL((gemm_pointwise_kernel<MT, KS, PB, false>), grid(PB), dim3(256), 0, st, g);
+  return check_hip(hipGetLastError(), "gemm_pointwise_kernel launch");
+}
+
 template <int MT, int NT>
 int launch_split(const GemmArgs& g, hipStream_t st) {
   // one workgroup per CU, each at least one step of 32 k per wavefront
@@ -409,6 +506,13 @@ int namsa_gemm_bf16(const float* A, long long sAb, long long sAi, long long sAk,
   if (split_k > 1 && sAk == 1 && sBk == 1 && M <= 64 && N <= 64) {
     if (M <= 32) return N <= 32 ? launch_split<1, 1>(g, st) : launch_split<1, 2>(g, st);
     return N <= 32 ? launch_split<2, 1>(g, st) : launch_split<2, 2>(g, st);
+  }
+  const long long buf_max = 0x7fffffffLL / 4;
+  if (batch == 1 && split_k == 1 && sBj == 1 && sCj == 1 && M <= 64 && K <= 64 && N >= 8192 && sBk >= N && sCi >= N &&
+      K * sBk <= buf_max && M * sCi <= buf_max) {
+    if (K <= 16) return M <= 32 ? launch_pointwise<1, 1>(g, st) : launch_pointwise<2, 1>(g, st);
+    if (K <= 32) return M <= 32 ? launch_pointwise<1, 2>(g, st) : launch_pointwise<2, 2>(g, st);
+    return M <= 32 ? launch_pointwise<1, 4>(g, st) : launch_pointwise<2, 4>(g, st);
   }
   if (N <= 32) return launch_gemm<4, 1>(g, st);
   if (M <= 32) return launch_gemm<1, 4>(g, st);
