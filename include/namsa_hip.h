@@ -375,6 +375,24 @@ int namsa_fno_layer(const void* x_in, const float* Zp, const void* fx, const voi
                     const float* Q1, const float* bq1, const float* Q2, const float* bq2, float* out, void* stream);
 
 /*
+ * The row-local work of the network's layers in training (32 channels, 2m = 32
+ * row-DFT columns), no counterpart in the reference.  x, pre_in, pre_out and
+ * out: float, channel-major [channels][B*H*W]; 32 channels must stay below
+ * 2 GiB.  Z, Zp, fx and fxT as above; Wt [32][cin], or
+ * [cin][32] if transposed.
+ *   lift:          out = Wt x + bias, cin <= 16                 (Zp, pre_in, pre_out NULL)
+ *   layer:         pre_out = alpha Fx Zp + Wt x + bias, out = gelu(pre_out)      (pre_in NULL)
+ *   layer backward: out = (alpha Fx Zp + Wt x) gelu'(pre_in)               (bias, pre_out NULL)
+ *   and with each  Z = zalpha * row DFT of out
+ *   last layer, first layer backward: out = alpha Fx Zp + Wt x [+ bias]
+ *                                                    (Z, pre_in, pre_out NULL, bias or NULL)
+ * The values are those of the separate products.
+ */
+int namsa_fno_rows(const float* x, int cin, const float* Zp, const void* fx, const void* fxT, const float* Wt,
+                   int transposed, const float* bias, float alpha, const float* pre_in, float* pre_out, float zalpha,
+                   int B, int H, int W, int Wp, float* out, float* Z, void* stream);
+
+/*
  * Spectral (one-shot) corrector: works on the centred exit spectrum Psi(k) of
  * the coarse path, |Psi|^2 being the CBED, inside the window
  * [r0, r0+H) x [c0, c0+W) of the Ny x Nx plane that bounds the bandwidth mask.

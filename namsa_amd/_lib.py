@@ -83,6 +83,8 @@ SIGNATURES = {
     "namsa_fno_lift": (_i, [_vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp]),
     "namsa_fno_layer": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                              _vp]),
+    "namsa_fno_rows": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _f, _vp, _vp, _f, _i, _i, _i, _i, _vp, _vp,
+                            _vp]),
     "namsa_modes_combine": (_i, [_vp, _vp, _i, _i, _i, _vp]),
     "namsa_modes_expand": (_i, [_vp, _vp, _i, _i, _i, _vp]),
 }

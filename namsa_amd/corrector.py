@@ -181,6 +181,7 @@ class FnoNet:
         self.gh = torch.empty((Hq, n), **f)
         self.ones = torch.empty(n, **f)
         call("namsa_fill", ptr(self.ones), n, np.float32(1.0), self.st)
+        self._row_tables()
         self.B = B
 
     def fused_ok(self):
@@ -197,14 +198,23 @@ class FnoNet:
         n = B * self.H * self.W
         self.xa = torch.empty((n, self.C), dtype=torch.bfloat16, device=self.device)
         self.xb = torch.empty((n, self.C), dtype=torch.bfloat16, device=self.device)
+        self._row_tables()
+        self.B_fused = B
+
+    def rows_ok(self, B):
+        """The row kernels of training are compiled for 32 channels and 16 modes and index 32 channels in 31 bits."""
+        return (self.C, self.m) == (32, 16) and self.cin <= 16 and 128 * B * self.H * self.W < 2 ** 31
+
+    def _row_tables(self):
+        """The row DFT in bf16, [Wp][2m] and transposed, zero from row W on."""
+        torch = _torch()
         if self.fx_bf is None:
             Wp = (self.W + 31) // 32 * 32
             fx = torch.zeros((Wp, 2 * self.m), dtype=torch.float32, device=self.device)
             fx[:self.W] = self.Fx
             self.Wp = Wp
-            self.fx_bf = fx.to(torch.bfloat16).contiguous()
             self.fxT_bf = fx.t().contiguous().to(torch.bfloat16)
-        self.B_fused = B
+            self.fx_bf = fx.to(torch.bfloat16).contiguous()
 
     # ------------------------------------------------------------------ GEMM
     def _gemm(self, A, sA, Bm, sB, Cm, sC, M, N, K, batch=1, split=1, alpha=1.0, beta=0.0, bias=None,
@@ -216,24 +226,37 @@ class FnoNet:
         return max(1, min(65535, K // 4096))
 
     def _spectral_forward(self, x, Xs, B, alpha):
-        """Xs[pq][(r,c)][b] = alpha * (Re, Im) of the centred m x m DFT modes of x [C][B*H*W]."""
+        """Xs[pq][(r,c)][b] = alpha * (Re, Im) of the centred m x m DFT modes of x [C][B*H*W]
+        (x None: Z already holds the row DFT, alpha included)."""
         H, W, C, m = self.H, self.W, self.C, self.m
         m2, CB = 2 * m, C * B
-        self._gemm(x, (0, W, 1), _addr(self.Fx), (0, m2, 1), _addr(self.Z), (0, m2, 1),
-                   CB * H, m2, W, alpha=alpha)
+        if x is not None:
+            self._gemm(x, (0, W, 1), _addr(self.Fx), (0, m2, 1), _addr(self.Z), (0, m2, 1),
+                       CB * H, m2, W, alpha=alpha)
         self._gemm(_addr(self.Fy), (0, H, 1), _addr(self.Z), (H * m2, m2, 1), _addr(self.Pm),
                    (m2 * m2, m2, 1), m2, m2, H, batch=CB)
         call("namsa_modes_combine", ptr(self.Pm), Xs, C, B, m, self.st)
+
+    def _spectral_rows(self, Ys, B):
+        """Zp = the row-inverse operand of the modes Ys."""
+        H, C, m = self.H, self.C, self.m
+        m2, CB = 2 * m, C * B
+        call("namsa_modes_expand", Ys, ptr(self.E), C, B, m, self.st)
+        self._gemm(_addr(self.Fy), (0, 1, H), _addr(self.E), (m2 * m2, m2, 1), _addr(self.Zp),
+                   (H * m2, m2, 1), H, m2, m2, batch=CB)
 
     def _spectral_inverse(self, Ys, dest, B, alpha, beta, gelu=False, P=None):
         """dest = alpha * Re(sum_modes Y e^{+i k.r}) + beta * dest (GELU optional)."""
         H, W, C, m = self.H, self.W, self.C, self.m
         m2, CB = 2 * m, C * B
-        call("namsa_modes_expand", Ys, ptr(self.E), C, B, m, self.st)
-        self._gemm(_addr(self.Fy), (0, 1, H), _addr(self.E), (m2 * m2, m2, 1), _addr(self.Zp),
-                   (H * m2, m2, 1), H, m2, m2, batch=CB)
+        self._spectral_rows(Ys, B)
         self._gemm(_addr(self.Zp), (0, m2, 1), _addr(self.Fx), (0, 1, m2), dest, (0, W, 1),
                    CB * H, W, m2, alpha=alpha, beta=beta, gelu=gelu, P=P)
+
+    def _rows(self, x, cin, Wt, transposed, B, out, Zp=None, bias=None, alpha=1.0, pre_in=None, pre_out=None, zalpha=1.0,
+              Z=None):
+        call("namsa_fno_rows", x, cin, Zp, ptr(self.fx_bf), ptr(self.fxT_bf), Wt, transposed, bias, np.float32(alpha), pre_in,
+             pre_out, np.float32(zalpha), B, self.H, self.W, self.Wp, out, Z, self.st)
 
     # ------------------------------------------------------------------ passes
     def forward(self, B):
@@ -242,17 +265,28 @@ class FnoNet:
         H, W, C, L, m, Hq = self.H, self.W, self.C, self.L, self.m, self.Hq
         n = B * H * W
         C2 = 2 * C
-        self._gemm(self._p("Wl"), (0, self.cin, 1), ptr(self.u), (0, n, 1), ptr(self.xs[0]), (0, n, 1),
-                   C, n, self.cin, bias=self._p("bl"), bias_mode=1)
+        rows = self.rows_ok(B)
+        if rows:
+            self._rows(ptr(self.u), self.cin, self._p("Wl"), 0, B, ptr(self.xs[0]), bias=self._p("bl"),
+                       Z=ptr(self.Z))
+        else:
+            self._gemm(self._p("Wl"), (0, self.cin, 1), ptr(self.u), (0, n, 1), ptr(self.xs[0]), (0, n, 1),
+                       C, n, self.cin, bias=self._p("bl"), bias_mode=1)
         for l in range(L):
             x = ptr(self.xs[l])
             Xs = _addr(self.Xs, l * m * m * C2 * B)
-            self._spectral_forward(x, Xs, B, 1.0)
+            self._spectral_forward(None if rows else x, Xs, B, 1.0)
             self._gemm(self._p("G", l), (C2 * C2, C2, 1), Xs, (C2 * B, B, 1), ptr(self.Ys), (C2 * B, B, 1),
                        C2, B, C2, batch=m * m)
+            last = l == L - 1
+            if rows:
+                self._spectral_rows(ptr(self.Ys), B)
+                self._rows(x, C, self._p("W", l), 0, B, ptr(self.xs[l + 1]), Zp=ptr(self.Zp),
+                           bias=self._p("b", l), alpha=1.0 / (H * W), pre_out=None if last else ptr(self.pre[l]),
+                           Z=None if last else ptr(self.Z))
+                continue
             self._gemm(self._p("W", l), (0, C, 1), x, (0, n, 1), ptr(self.xs[l + 1]), (0, n, 1), C, n, C,
                        bias=self._p("b", l), bias_mode=1)
-            last = l == L - 1
             self._spectral_inverse(ptr(self.Ys), ptr(self.xs[l + 1]), B, 1.0 / (H * W), 1.0,
                                    gelu=not last, P=None if last else ptr(self.pre[l]))
         self._gemm(self._p("Q1"), (0, C, 1), ptr(self.xs[L]), (0, n, 1), ptr(self.h), (0, n, 1), Hq, n, C,
@@ -348,8 +382,9 @@ class FnoNet:
         self._gemm(gh, (0, n, 1), ones, (0, 1, 0), self._g("bq1"), (0, 1, 1), Hq, 1, n, split=sp)
         ga, gb = self.ga, self.gb
         self._gemm(self._p("Q1"), (0, 1, C), gh, (0, n, 1), ptr(ga), (0, n, 1), C, n, Hq)
+        rows = self.rows_ok(B)
         for l in range(L - 1, -1, -1):
-            if l < L - 1:
+            if l < L - 1 and not rows:
                 call("namsa_gelu_backward", ptr(ga), ptr(self.pre[l]), C * n, self.st)
             g = ptr(ga)
             x = ptr(self.xs[l])
@@ -357,14 +392,20 @@ class FnoNet:
             self._gemm(g, (0, n, 1), ones, (0, 1, 0), self._g("b", l), (0, 1, 1), C, 1, n, split=sp)
             self._gemm(g, (0, n, 1), x, (0, 1, n), self._g("W", l), (0, C, 1), C, C, n, split=sp)
             # (dL/dRe Y, dL/dIm Y) = (Re, Im) DFT(gpre) / (H W)
-            self._spectral_forward(g, ptr(self.gYs), B, 1.0 / (H * W))
+            self._spectral_forward(None if rows and l < L - 1 else g, ptr(self.gYs), B, 1.0 / (H * W))
             self._gemm(ptr(self.gYs), (C2 * B, B, 1), Xs, (C2 * B, 1, B), self._g("G", l), (C2 * C2, C2, 1),
                        C2, C2, B, batch=m * m)
             self._gemm(self._p("G", l), (C2 * C2, 1, C2), ptr(self.gYs), (C2 * B, B, 1), ptr(self.Ys),
                        (C2 * B, B, 1), C2, B, C2, batch=m * m)
             # dL/dx = Re(sum gX e^{+i k.r}) + W^T gpre
-            self._spectral_inverse(ptr(self.Ys), ptr(gb), B, 1.0, 0.0)
-            self._gemm(self._p("W", l), (0, 1, C), g, (0, n, 1), ptr(gb), (0, n, 1), C, n, C, beta=1.0)
+            if rows:  # and on to the layer before: its gpre and the row DFT of that
+                self._spectral_rows(ptr(self.Ys), B)
+                self._rows(g, C, self._p("W", l), 1, B, ptr(gb), Zp=ptr(self.Zp),
+                           pre_in=ptr(self.pre[l - 1]) if l else None, zalpha=1.0 / (H * W),
+                           Z=ptr(self.Z) if l else None)
+            else:
+                self._spectral_inverse(ptr(self.Ys), ptr(gb), B, 1.0, 0.0)
+                self._gemm(self._p("W", l), (0, 1, C), g, (0, n, 1), ptr(gb), (0, n, 1), C, n, C, beta=1.0)
             ga, gb = gb, ga
         g = ptr(ga)
         self._gemm(g, (0, n, 1), ptr(self.u), (0, 1, n), self._g("Wl"), (0, self.cin, 1), C, self.cin, n,

@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "gelu.hpp"
 #include "namsa_hip.h"
 #include "passes.hpp"  // wave_sum
 
@@ -14,12 +15,6 @@ namespace namsa {
 
 __global__ void fill_kernel(float* __restrict__ x, long long n, float v) {
   for (long long i = blockIdx.x * 256LL + threadIdx.x; i < n; i += 256LL * gridDim.x) x[i] = v;
-}
-
-__device__ __forceinline__ float gelu_grad_tanh(float x) {
-  const float c = 0.7978845608028654f;
-  const float t = tanhf(c * (x + 0.044715f * x * x * x));
-  return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * c * (1.0f + 3.0f * 0.044715f * x * x);
 }
 
 __global__ void gelu_backward_kernel(float* __restrict__ g, const float* __restrict__ pre, long long n) {

@@ -29,6 +29,7 @@
 #include <cstdint>
 
 #include "common.hpp"
+#include "gelu.hpp"
 #include "namsa_hip.h"
 
 namespace namsa {
@@ -54,11 +55,6 @@ struct GemmArgs {
 
 constexpr int kTK = 32;
 constexpr int kLdK = kTK + 8;  // LDS row pitch in bf16: 80 bytes keeps every row 16-byte aligned
-
-__device__ __forceinline__ float gelu_tanh(float x) {
-  const float c = 0.7978845608028654f;  // sqrt(2/pi)
-  return 0.5f * x * (1.0f + tanhf(c * (x + 0.044715f * x * x * x)));
-}
 
 // Four consecutive floats at any 4-byte aligned address, one 16-byte load.
 struct alignas(4) F4 {
