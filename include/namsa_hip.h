@@ -393,6 +393,19 @@ int namsa_fno_rows(const float* x, int cin, const float* Zp, const void* fx, con
                    int B, int H, int W, int Wp, float* out, float* Z, void* stream);
 
 /*
+ * The network's head in training (32 -> 64 -> 2 channels), no counterpart in
+ * the reference; x, out, gout and gx float channel-major [channels][n], 32
+ * channels below 2 GiB, Q1 [64][32], Q2 [2][64].
+ *   namsa_fno_head:          out = Q2 gelu(Q1 x + bq1) + bq2
+ *   namsa_fno_head_backward: gx = d(sum out gout) / dx; the gradients of the
+ *                            weights are added to gQ1, gbq1, gQ2 and gbq2
+ */
+int namsa_fno_head(const float* x, const float* Q1, const float* bq1, const float* Q2, const float* bq2, long long n,
+                   float* out, void* stream);
+int namsa_fno_head_backward(const float* x, const float* Q1, const float* bq1, const float* Q2, const float* gout,
+                            long long n, float* gx, float* gQ1, float* gbq1, float* gQ2, float* gbq2, void* stream);
+
+/*
  * Spectral (one-shot) corrector: works on the centred exit spectrum Psi(k) of
  * the coarse path, |Psi|^2 being the CBED, inside the window
  * [r0, r0+H) x [c0, c0+W) of the Ny x Nx plane that bounds the bandwidth mask.

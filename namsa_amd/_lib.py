@@ -85,6 +85,8 @@ SIGNATURES = {
                              _vp]),
     "namsa_fno_rows": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _f, _vp, _vp, _f, _i, _i, _i, _i, _vp, _vp,
                             _vp]),
+    "namsa_fno_head": (_i, [_vp, _vp, _vp, _vp, _vp, _ll, _vp, _vp]),
+    "namsa_fno_head_backward": (_i, [_vp, _vp, _vp, _vp, _vp, _ll, _vp, _vp, _vp, _vp, _vp, _vp]),
     "namsa_modes_combine": (_i, [_vp, _vp, _i, _i, _i, _vp]),
     "namsa_modes_expand": (_i, [_vp, _vp, _i, _i, _i, _vp]),
 }

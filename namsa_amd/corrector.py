@@ -174,11 +174,9 @@ class FnoNet:
         f = dict(dtype=torch.float32, device=self.device)
         self.xs = [torch.empty((C, n), **f) for _ in range(L + 1)]
         self.pre = [torch.empty((C, n), **f) for _ in range(L - 1)]
-        self.hpre = torch.empty((Hq, n), **f)
-        self.h = torch.empty((Hq, n), **f)
         self.ga = torch.empty((C, n), **f)
         self.gb = torch.empty((C, n), **f)
-        self.gh = torch.empty((Hq, n), **f)
+        self.hpre = self.h = self.gh = None
         self.ones = torch.empty(n, **f)
         call("namsa_fill", ptr(self.ones), n, np.float32(1.0), self.st)
         self._row_tables()
@@ -204,6 +202,17 @@ class FnoNet:
     def rows_ok(self, B):
         """The row kernels of training are compiled for 32 channels and 16 modes and index 32 channels in 31 bits."""
         return (self.C, self.m) == (32, 16) and self.cin <= 16 and 128 * B * self.H * self.W < 2 ** 31
+
+    def head_ok(self, B):
+        """The head's kernels of training are compiled for 32 and 64 channels and index 32 channels in 31 bits."""
+        return (self.C, self.Hq) == (32, 64) and 128 * B * self.H * self.W < 2 ** 31
+
+    def _ensure_hidden(self, n):
+        """The head's hidden activation, pre-activation and gradient (the head kernels keep none)."""
+        if self.h is None or self.h.shape[1] < n:
+            torch = _torch()
+            self.hpre, self.h, self.gh = (torch.empty((self.Hq, n), dtype=torch.float32, device=self.device)
+                                          for _ in range(3))
 
     def _row_tables(self):
         """The row DFT in bf16, [Wp][2m] and transposed, zero from row W on."""
@@ -289,6 +298,11 @@ class FnoNet:
                        bias=self._p("b", l), bias_mode=1)
             self._spectral_inverse(ptr(self.Ys), ptr(self.xs[l + 1]), B, 1.0 / (H * W), 1.0,
                                    gelu=not last, P=None if last else ptr(self.pre[l]))
+        if self.head_ok(B):
+            call("namsa_fno_head", ptr(self.xs[L]), self._p("Q1"), self._p("bq1"), self._p("Q2"), self._p("bq2"), n,
+                 ptr(self.out), self.st)
+            return self.out
+        self._ensure_hidden(n)
         self._gemm(self._p("Q1"), (0, C, 1), ptr(self.xs[L]), (0, n, 1), ptr(self.h), (0, n, 1), Hq, n, C,
                    bias=self._p("bq1"), bias_mode=1, gelu=True, P=ptr(self.hpre))
         self._gemm(self._p("Q2"), (0, Hq, 1), ptr(self.h), (0, n, 1), ptr(self.out), (0, n, 1), 2, n, Hq,
@@ -373,15 +387,19 @@ class FnoNet:
         sp = self._split(n)
         call("namsa_fill", ptr(self.grad), self.n_params, np.float32(0.0), self.st)
         go, ones = ptr(self.gout), ptr(self.ones)
-        self._gemm(go, (0, n, 1), ptr(self.h), (0, 1, n), self._g("Q2"), (0, Hq, 1), 2, Hq, n, split=sp)
-        self._gemm(go, (0, n, 1), ones, (0, 1, 0), self._g("bq2"), (0, 1, 1), 2, 1, n, split=sp)
-        self._gemm(self._p("Q2"), (0, 1, Hq), go, (0, n, 1), ptr(self.gh), (0, n, 1), Hq, n, 2)
-        call("namsa_gelu_backward", ptr(self.gh), ptr(self.hpre), Hq * n, self.st)
-        gh = ptr(self.gh)
-        self._gemm(gh, (0, n, 1), ptr(self.xs[L]), (0, 1, n), self._g("Q1"), (0, C, 1), Hq, C, n, split=sp)
-        self._gemm(gh, (0, n, 1), ones, (0, 1, 0), self._g("bq1"), (0, 1, 1), Hq, 1, n, split=sp)
         ga, gb = self.ga, self.gb
-        self._gemm(self._p("Q1"), (0, 1, C), gh, (0, n, 1), ptr(ga), (0, n, 1), C, n, Hq)
+        if self.head_ok(B):
+            call("namsa_fno_head_backward", ptr(self.xs[L]), self._p("Q1"), self._p("bq1"), self._p("Q2"), go, n, ptr(ga),
+                 self._g("Q1"), self._g("bq1"), self._g("Q2"), self._g("bq2"), self.st)
+        else:
+            self._gemm(go, (0, n, 1), ptr(self.h), (0, 1, n), self._g("Q2"), (0, Hq, 1), 2, Hq, n, split=sp)
+            self._gemm(go, (0, n, 1), ones, (0, 1, 0), self._g("bq2"), (0, 1, 1), 2, 1, n, split=sp)
+            self._gemm(self._p("Q2"), (0, 1, Hq), go, (0, n, 1), ptr(self.gh), (0, n, 1), Hq, n, 2)
+            call("namsa_gelu_backward", ptr(self.gh), ptr(self.hpre), Hq * n, self.st)
+            gh = ptr(self.gh)
+            self._gemm(gh, (0, n, 1), ptr(self.xs[L]), (0, 1, n), self._g("Q1"), (0, C, 1), Hq, C, n, split=sp)
+            self._gemm(gh, (0, n, 1), ones, (0, 1, 0), self._g("bq1"), (0, 1, 1), Hq, 1, n, split=sp)
+            self._gemm(self._p("Q1"), (0, 1, C), gh, (0, n, 1), ptr(ga), (0, n, 1), C, n, Hq)
         rows = self.rows_ok(B)
         for l in range(L - 1, -1, -1):
             if l < L - 1 and not rows:

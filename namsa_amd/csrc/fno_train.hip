@@ -42,6 +42,14 @@ constexpr int kNowhere = 0x7ffffffc;    // a byte offset past every buffer: stor
 
 __device__ __forceinline__ bf16x8 ld8(const __bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
+// A wavefront exchanges through its own LDS tile in program order: only the
+// compiler has to be held to it.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
@@ -271,6 +279,251 @@ int launch_rows(const RowArgs& g, hipStream_t st) {
   return check_hip(hipGetLastError(), "fno_rows_kernel launch");
 }
 
+// ------------------------------------------------------------------ the head
+// out = Q2 gelu(Q1 x + bq1) + bq2, 32 -> 64 -> 2 channels, and its gradients.
+// The hidden activation, 64 floats a pixel, is never stored: the backward pass
+// forms it again from x, 12 MFLOP of matrix products for each 118 MB (16 images
+// of 170 x 170) that hidden value, pre-activation and gradient took each time
+// they were written or read.  At that size, as products of their own -> here:
+// forward 129 -> 32 us, backward 340 -> 80 us, and 355 MB less held.
+
+constexpr int kHid = 64;
+constexpr int kOut = 2;
+constexpr int kHeadTiles = 4;             // 32-pixel tiles of a forward wavefront
+constexpr int kHeadWaves = 8;             // wavefronts of a backward workgroup
+constexpr int kHPitch = kHid + 8;         // LDS row pitch in bf16 (144 bytes: 16-byte aligned rows)
+
+struct HeadArgs {
+  const float* x;                         // [32][n]
+  const float *Q1, *bq1, *Q2, *bq2;       // [64][32], [64], [2][64], [2]
+  int n;
+  float* out;                             // [2][n]
+  const float* gout;                      // [2][n]
+  float *gx, *gQ1, *gbq1, *gQ2, *gbq2;
+};
+
+__device__ __forceinline__ Rsrc buffer_of(const void* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, kRawBuffer);
+}
+
+// 16 channels' steps of a tile, channels 16 s + 8 half + e at this lane's pixel
+__device__ __forceinline__ void load_pixels(float (&v)[2][8], Rsrc r, int pitch, int px, int n, int kh) {
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[s][e] = load_b32(r, px < n ? kh * pitch + 4 * px : kNowhere, (16 * s + e) * pitch);
+}
+
+__device__ __forceinline__ void round_pixels(bf16x8 (&b)[2], const float (&v)[2][8]) {
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) b[s][e] = __bf16(v[s][e]);
+}
+
+// Forward: bound by the 64 tanh of a pixel (about 45 instructions each).  The
+// hidden block leaves the matrix cores with its pixel in the lane and 4 of
+// every 8 units in each half of the wavefront; exchanging half the registers
+// between the halves makes it the next product's operand, no LDS.
+__global__ void __launch_bounds__(256) fno_head_kernel(HeadArgs g) {
+  const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5, kh = 8 * half;
+  const int pitch = 4 * g.n;
+  const Rsrc rx = buffer_of(g.x, kCh * pitch), ro = buffer_of(g.out, kOut * pitch);
+  const Rsrc rq1 = buffer_of(g.Q1, 4 * kHid * kCh), rq2 = buffer_of(g.Q2, 4 * kOut * kHid);
+  const Rsrc rb1 = buffer_of(g.bq1, 4 * kHid);
+  const int first = 32 * kHeadTiles * (blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+  bf16x8 q1[2][2], q2[4];  // rows j of Q1, rows t of Q2
+  float b1[2][16];
+#pragma unroll
+  for (int jb = 0; jb < 2; ++jb) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) q1[jb][s] = load_f8(rq1, 4 * (col * kCh + kh), 4 * (32 * jb * kCh + 16 * s));
+#pragma unroll
+    for (int i = 0; i < 16; ++i) b1[jb][i] = load_b32(rb1, 16 * half, 4 * (32 * jb + 8 * (i >> 2) + (i & 3)));
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s) q2[s] = load_f8(rq2, col < kOut ? 4 * (col * kHid + kh) : kNowhere, 64 * s);
+  const float b2[kOut] = {g.bq2[0], g.bq2[1]};
+  float next[2][8];
+  load_pixels(next, rx, pitch, first + col, g.n, kh);
+  for (int t = 0; t < kHeadTiles; ++t) {
+    const int x0 = first + 32 * t, px = x0 + col;
+    if (x0 >= g.n) return;
+    bf16x8 bx[2];
+    round_pixels(bx, next);
+    if (t + 1 < kHeadTiles) load_pixels(next, rx, pitch, px + 32, g.n, kh);
+    f32x16 out = zero16();
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) {
+      f32x16 acc = zero16();
+#pragma unroll
+      for (int s = 0; s < 2; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q1[jb][s], bx[s], acc, 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        bf16x8 h;  // units 16 s + (0..3, 8..11 in the lower half; 4..7, 12..15 in the upper)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) h[e] = __bf16(gelu_tanh(acc[8 * s + e] + b1[jb][8 * s + e]));
+        u32x4 w = __builtin_bit_cast(u32x4, h);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const auto p = __builtin_amdgcn_permlane32_swap(w[e], w[e + 2], false, false);
+          w[e] = p[0];
+          w[e + 2] = p[1];
+        }
+        out = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q2[2 * jb + s], __builtin_bit_cast(bf16x8, w), out, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < kOut; ++c) store_b32(out[c] + b2[c], ro, half == 0 && px < g.n ? 4 * px : kNowhere, c * pitch);
+  }
+}
+
+// Backward, one workgroup a CU, its wavefronts striding over the tiles with the
+// weight gradients in their accumulators.  The hidden block is formed with its
+// unit in the lane and 16 pixels in the registers: that is the operand of
+// dQ1 = gh x^T, of dQ2 and of dbq1 as it stands (x and gout read once more, a
+// channel a lane, the pixels in the registers' order).  Only gh goes through
+// LDS, to become the operand of gx = Q1^T gh.  Bound by the 64 tanh of a pixel
+// (one for value and derivative: two took 99 us) and the arithmetic around them.
+__global__ void __launch_bounds__(64 * kHeadWaves, 2) fno_head_backward_kernel(HeadArgs g) {
+  __shared__ __align__(16) __bf16 tt_all[kHeadWaves][32][kHPitch];
+  __shared__ float red[kHid * kCh + kHid + kOut * kHid + kOut];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 31, half = lane >> 5, kh = 8 * half;
+  __bf16 (*tt)[kHPitch] = tt_all[wave];
+  const int pitch = 4 * g.n;
+  const Rsrc rx = buffer_of(g.x, kCh * pitch), rg = buffer_of(g.gout, kOut * pitch), ro = buffer_of(g.gx, kCh * pitch);
+  const Rsrc rq1 = buffer_of(g.Q1, 4 * kHid * kCh), rq2 = buffer_of(g.Q2, 4 * kOut * kHid);
+  bf16x8 q1[2][2], q1t[4], q2[2];  // Q1 rows j; Q1^T rows c; Q2^T rows j
+  float b1[2];
+#pragma unroll
+  for (int jb = 0; jb < 2; ++jb) {
+    b1[jb] = g.bq1[32 * jb + col];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) q1[jb][s] = load_f8(rq1, 4 * (col * kCh + kh), 4 * (32 * jb * kCh + 16 * s));
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      q2[jb][e] = __bf16(e < kOut ? load_b32(rq2, half == 0 ? 4 * col : kNowhere, 4 * (e * kHid + 32 * jb)) : 0.0f);
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q1t[s][e] = __bf16(load_b32(rq1, 4 * (kh * kCh + col), 4 * (16 * s + e) * kCh));
+
+  bf16x8 ones;  // row kOut of an operand: sums the other over its pixels
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ones[e] = __bf16(col == kOut ? 1.0f : 0.0f);
+  f32x16 gq1[2] = {zero16(), zero16()}, gq2[2] = {zero16(), zero16()};  // gq2: rows of dQ2, then dbq1
+  float gb2[kOut] = {0.0f, 0.0f};
+  const int step = 32 * kHeadWaves * gridDim.x;
+  int x0 = 32 * (kHeadWaves * blockIdx.x + wave);
+  float next[2][8];
+  load_pixels(next, rx, pitch, x0 + col, g.n, kh);
+  for (; x0 < g.n; x0 += step) {
+    const int px = x0 + col;
+    bf16x8 bx[2], go, gt[2], xt[2];
+    round_pixels(bx, next);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) go[e] = __bf16(0.0f);
+#pragma unroll
+    for (int c = 0; c < kOut; ++c) {
+      go[c] = __bf16(load_b32(rg, half == 0 && px < g.n ? 4 * px : kNowhere, c * pitch));
+      gb2[c] += static_cast<float>(go[c]);
+    }
+    // a channel of x, or a row of gout, to a lane, at the hidden block's pixels
+    // in register order: 8 (i / 4) + 4 half + i % 4
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int p = x0 + 8 * i + 4 * half;
+      u32x4 xv, gv;
+      if (x0 + 32 <= g.n) {
+        xv = __builtin_amdgcn_raw_buffer_load_b128(rx, col * pitch + 4 * p, 0, 0);
+        gv = __builtin_amdgcn_raw_buffer_load_b128(rg, col < kOut ? col * pitch + 4 * p : kNowhere, 0, 0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool in = p + e < g.n;
+          xv[e] = __builtin_amdgcn_raw_buffer_load_b32(rx, in ? col * pitch + 4 * (p + e) : kNowhere, 0, 0);
+          gv[e] = __builtin_amdgcn_raw_buffer_load_b32(rg, in && col < kOut ? col * pitch + 4 * (p + e) : kNowhere, 0,
+                                                       0);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        xt[i >> 1][4 * (i & 1) + e] = __bf16(__builtin_bit_cast(float, static_cast<unsigned>(xv[e])));
+        gt[i >> 1][4 * (i & 1) + e] = __bf16(__builtin_bit_cast(float, static_cast<unsigned>(gv[e])));
+      }
+    }
+    load_pixels(next, rx, pitch, px + step, g.n, kh);
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) {
+      f32x16 pre = zero16();
+#pragma unroll
+      for (int s = 0; s < 2; ++s) pre = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bx[s], q1[jb][s], pre, 0, 0, 0);
+      const f32x16 gh0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(go, q2[jb], zero16(), 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        bf16x8 h, gh;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int i = 8 * s + e;
+          const float v = pre[i] + b1[jb], t = gelu_t(v);
+          h[e] = __bf16(gelu_tanh(v, t));
+          gh[e] = __bf16(gh0[i] * gelu_grad_tanh(v, t));
+          tt[8 * (i >> 2) + 4 * half + (i & 3)][32 * jb + col] = gh[e];
+        }
+        gq1[jb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gh, xt[s], gq1[jb], 0, 0, 0);
+        gq2[jb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gt[s], h, gq2[jb], 0, 0, 0);
+        gq2[jb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, gh, gq2[jb], 0, 0, 0);
+      }
+    }
+    wave_sync();
+    f32x16 gx = zero16();
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      gx = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q1t[s], ld8(&tt[col][16 * s + kh]), gx, 0, 0, 0);
+    wave_sync();
+    const int at = px < g.n ? 4 * half * pitch + 4 * px : kNowhere;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) store_b32(gx[i], ro, at, (8 * (i >> 2) + (i & 3)) * pitch);
+  }
+
+  // the workgroup's sums, then one atomic a value
+  constexpr int kB1 = kHid * kCh, kQ2 = kB1 + kHid, kB2 = kQ2 + kOut * kHid, kAll = kB2 + kOut;
+  for (int i = threadIdx.x; i < kAll; i += 64 * kHeadWaves) red[i] = 0.0f;
+  __syncthreads();
+#pragma unroll
+  for (int jb = 0; jb < 2; ++jb) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      atomicAdd(&red[(32 * jb + 8 * (i >> 2) + 4 * half + (i & 3)) * kCh + col], gq1[jb][i]);
+    if (half == 0) {
+#pragma unroll
+      for (int c = 0; c < kOut; ++c) atomicAdd(&red[kQ2 + c * kHid + 32 * jb + col], gq2[jb][c]);
+      atomicAdd(&red[kB1 + 32 * jb + col], gq2[jb][kOut]);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < kOut; ++c) {
+    float v = gb2[c];  // the upper half's is 0
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (lane == 0) atomicAdd(&red[kB2 + c], v);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kAll; i += 64 * kHeadWaves) {
+    float* dst = i < kB1 ? g.gQ1 + i : i < kQ2 ? g.gbq1 + (i - kB1) : i < kB2 ? g.gQ2 + (i - kQ2) : g.gbq2 + (i - kB2);
+    atomicAdd(dst, red[i]);
+  }
+}
+
+int head_size_ok(long long n, const char* who) {
+  if (n <= 0 || n > 0x7fffffffLL / (4 * kCh))
+    return fail(kErrArg, "%s: n=%lld pixels (32 channels must stay below 2 GiB)", who, n);
+  return kOk;
+}
+
 }  // namespace
 }  // namespace namsa
 
@@ -300,6 +553,27 @@ int namsa_fno_rows(const float* x, int cin, const float* Zp, const void* fx, con
   if (Zp && !Z && none && bias && !transposed) return launch_rows<2, true, false, true, kPlain, false>(g, st);
   if (Zp && !Z && none && !bias && transposed) return launch_rows<2, true, true, false, kPlain, false>(g, st);
   return fail(kErrArg, "namsa_fno_rows: no layer has this combination of Zp, Z, bias, pre_in and pre_out");
+}
+
+int namsa_fno_head(const float* x, const float* Q1, const float* bq1, const float* Q2, const float* bq2, long long n,
+                   float* out, void* stream) {
+  if (int rc = head_size_ok(n, "namsa_fno_head")) return rc;
+  if (!x || !Q1 || !bq1 || !Q2 || !bq2 || !out) return fail(kErrArg, "namsa_fno_head: null argument");
+  const HeadArgs g{x, Q1, bq1, Q2, bq2, static_cast<int>(n), out, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  const int per = 4 * 32 * kHeadTiles;
+  hipLaunchKernelGGL(fno_head_kernel, dim3((g.n + per - 1) / per), dim3(256), 0, as_stream(stream), g);
+  return check_hip(hipGetLastError(), "fno_head_kernel launch");
+}
+
+int namsa_fno_head_backward(const float* x, const float* Q1, const float* bq1, const float* Q2, const float* gout,
+                            long long n, float* gx, float* gQ1, float* gbq1, float* gQ2, float* gbq2, void* stream) {
+  if (int rc = head_size_ok(n, "namsa_fno_head_backward")) return rc;
+  if (!x || !Q1 || !bq1 || !Q2 || !gout || !gx || !gQ1 || !gbq1 || !gQ2 || !gbq2)
+    return fail(kErrArg, "namsa_fno_head_backward: null argument");
+  const HeadArgs g{x, Q1, bq1, Q2, nullptr, static_cast<int>(n), nullptr, gout, gx, gQ1, gbq1, gQ2, gbq2};
+  const int per = 32 * kHeadWaves, groups = std::min((g.n + per - 1) / per, device_cu_count());
+  hipLaunchKernelGGL(fno_head_backward_kernel, dim3(groups), dim3(64 * kHeadWaves), 0, as_stream(stream), g);
+  return check_hip(hipGetLastError(), "fno_head_backward_kernel launch");
 }
 
 }  // extern "C"
