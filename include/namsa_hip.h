@@ -375,6 +375,13 @@ int namsa_fno_layer(const void* x_in, const float* Zp, const void* fx, const voi
                     const float* Q1, const float* bq1, const float* Q2, const float* bq2, float* out, void* stream);
 
 /*
+ * A pointwise layer's weight gradients, gW[M][N] += gy x^T and gb[M] += row
+ * sums of gy, from gy [M][n] and x [N][n] (M, N <= 32) rounded to bf16, FP32
+ * sums.
+ */
+int namsa_weight_grad(const float* gy, const float* x, long long n, int M, int N, float* gW, float* gb, void* stream);
+
+/*
  * The row-local work of the network's layers in training (32 channels, 2m = 32
  * row-DFT columns), no counterpart in the reference.  x, pre_in, pre_out and
  * out: float, channel-major [channels][B*H*W]; 32 channels must stay below

@@ -83,6 +83,7 @@ SIGNATURES = {
     "namsa_fno_lift": (_i, [_vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp]),
     "namsa_fno_layer": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                              _vp]),
+    "namsa_weight_grad": (_i, [_vp, _vp, _ll, _i, _i, _vp, _vp, _vp]),
     "namsa_fno_rows": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _f, _vp, _vp, _f, _i, _i, _i, _i, _vp, _vp,
                             _vp]),
     "namsa_fno_head": (_i, [_vp, _vp, _vp, _vp, _vp, _ll, _vp, _vp]),

@@ -234,6 +234,15 @@ class FnoNet:
     def _split(self, K):
         return max(1, min(65535, K // 4096))
 
+    def _weight_grad(self, g, x, n, N, gW, gb):
+        """gW += g x^T and gb += row sums of g, for g [C][n] and x [N][n]."""
+        if self.C <= 32 and N <= 32:
+            call("namsa_weight_grad", g, x, n, self.C, N, gW, gb, self.st)
+            return
+        sp = self._split(n)
+        self._gemm(g, (0, n, 1), x, (0, 1, n), gW, (0, N, 1), self.C, N, n, split=sp)
+        self._gemm(g, (0, n, 1), ptr(self.ones), (0, 1, 0), gb, (0, 1, 1), self.C, 1, n, split=sp)
+
     def _spectral_forward(self, x, Xs, B, alpha):
         """Xs[pq][(r,c)][b] = alpha * (Re, Im) of the centred m x m DFT modes of x [C][B*H*W]
         (x None: Z already holds the row DFT, alpha included)."""
@@ -407,8 +416,7 @@ class FnoNet:
             g = ptr(ga)
             x = ptr(self.xs[l])
             Xs = _addr(self.Xs, l * m * m * C2 * B)
-            self._gemm(g, (0, n, 1), ones, (0, 1, 0), self._g("b", l), (0, 1, 1), C, 1, n, split=sp)
-            self._gemm(g, (0, n, 1), x, (0, 1, n), self._g("W", l), (0, C, 1), C, C, n, split=sp)
+            self._weight_grad(g, x, n, C, self._g("W", l), self._g("b", l))
             # (dL/dRe Y, dL/dIm Y) = (Re, Im) DFT(gpre) / (H W)
             self._spectral_forward(None if rows and l < L - 1 else g, ptr(self.gYs), B, 1.0 / (H * W))
             self._gemm(ptr(self.gYs), (C2 * B, B, 1), Xs, (C2 * B, 1, B), self._g("G", l), (C2 * C2, C2, 1),
@@ -426,9 +434,7 @@ class FnoNet:
                 self._gemm(self._p("W", l), (0, 1, C), g, (0, n, 1), ptr(gb), (0, n, 1), C, n, C, beta=1.0)
             ga, gb = gb, ga
         g = ptr(ga)
-        self._gemm(g, (0, n, 1), ptr(self.u), (0, 1, n), self._g("Wl"), (0, self.cin, 1), C, self.cin, n,
-                   split=sp)
-        self._gemm(g, (0, n, 1), ones, (0, 1, 0), self._g("bl"), (0, 1, 1), C, 1, n, split=sp)
+        self._weight_grad(g, ptr(self.u), n, self.cin, self._g("Wl"), self._g("bl"))
 
     def adam(self, lr, b1=0.9, b2=0.999, eps=1e-8, wd=0.0):
         self.adam_step += 1

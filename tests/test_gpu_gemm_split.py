@@ -41,3 +41,20 @@ def test_split_products(gpu, M, N, K, batch, pad, off, zero):
         err = np.linalg.norm(got[at] - C0[at] - 0.5 * (a @ w.T)) / np.linalg.norm(np.abs(a) @ np.abs(w).T)
         assert err < 2e-5, (b, err)
     assert np.array_equal(got[~touched], C0[~touched])
+
+
+@pytest.mark.parametrize("M,N,n", [(1, 1, 1), (32, 32, 31), (8, 3, 127), (32, 7, 129), (32, 32, 70001)])
+def test_weight_grad(gpu, M, N, n):
+    """The product with its row sums, both added to what is there; the same bound."""
+    import torch
+
+    print(f"weight grad M={M} N={N} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    gy, x = (rng.standard_normal((k, n)).astype(np.float32) for k in (M, N))
+    C0 = rng.standard_normal((M, N + 1)).astype(np.float32)
+    gd, xd, W, b = (torch.from_numpy(v.copy()).to(gpu) for v in (gy, x, C0[:, :N], C0[:, N]))
+    L.call("namsa_weight_grad", L.ptr(gd), L.ptr(xd), n, M, N, L.ptr(W), L.ptr(b), L.stream_handle())
+    got = np.concatenate([W.cpu().numpy(), b.cpu().numpy()[:, None]], 1).astype(np.float64)
+    a, w = bf16(gy), np.concatenate([bf16(x), np.ones((1, n))])
+    err = np.linalg.norm(got - C0 - a @ w.T) / np.linalg.norm(np.abs(a) @ np.abs(w).T)
+    assert err < 2e-5, err
