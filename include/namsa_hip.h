@@ -354,6 +354,14 @@ int namsa_adam(float* p, const float* g, float* m, float* v, long long n, float 
 int namsa_modes_combine(const float* P, float* Xs, int C, int B, int m, void* stream);
 int namsa_modes_expand(const float* Ys, float* E, int C, int B, int m, void* stream);
 /*
+ * The y transforms of m = 16 modes with the bookkeeping above in one kernel
+ * each, the values of the separate products: Xs from Z and Zp from Ys (Z, Zp
+ * float [(c*B + b)*H + y][32]).  fy: bf16 [32][Hp] = Fy[(r,p)][y] (columns >= H
+ * zero), fyT: bf16 [Hp][32] its transpose; Hp a multiple of 32, >= H.
+ */
+int namsa_modes_forward(const float* Z, const void* fy, int H, int Hp, int C, int B, float* Xs, void* stream);
+int namsa_modes_inverse(const float* Ys, const void* fyT, int H, int Hp, int C, int B, float* Zp, void* stream);
+/*
  * Channel-last BF16 inference of the corrector network (32 channels, 2m = 32
  * row-DFT columns, head width 64), no counterpart in the reference.
  * Activations x: bf16 [B*H][W][32]; Z / Zp: float [(c*B + b)*H + y][32] (the

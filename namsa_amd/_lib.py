@@ -88,6 +88,8 @@ SIGNATURES = {
                             _vp]),
     "namsa_fno_head": (_i, [_vp, _vp, _vp, _vp, _vp, _ll, _vp, _vp]),
     "namsa_fno_head_backward": (_i, [_vp, _vp, _vp, _vp, _vp, _ll, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "namsa_modes_forward": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _vp]),
+    "namsa_modes_inverse": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _vp]),
     "namsa_modes_combine": (_i, [_vp, _vp, _i, _i, _i, _vp]),
     "namsa_modes_expand": (_i, [_vp, _vp, _i, _i, _i, _vp]),
 }

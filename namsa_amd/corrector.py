@@ -81,7 +81,7 @@ class FnoNet:
         self.B = 0                  # samples the training buffers hold
         self.B_common = 0           # ... the mode-space and input / output buffers
         self.B_fused = 0            # ... the channel-last inference buffers
-        self.fx_bf = None
+        self.fx_bf = self.fy_bf = None
         self._graphs = {}           # B -> captured forward_fused
 
     # ------------------------------------------------------------------ parameters
@@ -161,6 +161,12 @@ class FnoNet:
         self.E = torch.empty((C * B, 2 * m, 2 * m), **f)
         self.Zp = torch.empty((C * B * H, 2 * m), **f)
         self.sums = torch.empty(2 * B, dtype=torch.float64, device=self.device)
+        if self.m == 16 and self.fy_bf is None:    # the y transform in bf16, [2m][Hp] and transposed, zero from H on
+            self.Hp = (H + 31) // 32 * 32
+            fy = torch.zeros((2 * m, self.Hp), dtype=torch.float32, device=self.device)
+            fy[:, :H] = self.Fy
+            self.fyT_bf = fy.t().contiguous().to(torch.bfloat16)
+            self.fy_bf = fy.to(torch.bfloat16).contiguous()
         self.B_common = B
 
     def ensure(self, B):
@@ -251,6 +257,15 @@ class FnoNet:
         if x is not None:
             self._gemm(x, (0, W, 1), _addr(self.Fx), (0, m2, 1), _addr(self.Z), (0, m2, 1),
                        CB * H, m2, W, alpha=alpha)
+        self._y_forward(Xs, B)
+
+    def _y_forward(self, Xs, B):
+        """Xs = the modes of the row DFT in Z."""
+        H, C, m = self.H, self.C, self.m
+        m2, CB = 2 * m, C * B
+        if m == 16 and CB >= 64:   # fewer items: the strided product sums over y in another order
+            call("namsa_modes_forward", ptr(self.Z), ptr(self.fy_bf), H, self.Hp, C, B, Xs, self.st)
+            return
         self._gemm(_addr(self.Fy), (0, H, 1), _addr(self.Z), (H * m2, m2, 1), _addr(self.Pm),
                    (m2 * m2, m2, 1), m2, m2, H, batch=CB)
         call("namsa_modes_combine", ptr(self.Pm), Xs, C, B, m, self.st)
@@ -259,6 +274,9 @@ class FnoNet:
         """Zp = the row-inverse operand of the modes Ys."""
         H, C, m = self.H, self.C, self.m
         m2, CB = 2 * m, C * B
+        if m == 16 and H > 32:     # fewer rows: the strided product sums the two parts in another order
+            call("namsa_modes_inverse", Ys, ptr(self.fyT_bf), H, self.Hp, C, B, ptr(self.Zp), self.st)
+            return
         call("namsa_modes_expand", Ys, ptr(self.E), C, B, m, self.st)
         self._gemm(_addr(self.Fy), (0, 1, H), _addr(self.E), (m2 * m2, m2, 1), _addr(self.Zp),
                    (H * m2, m2, 1), H, m2, m2, batch=CB)
@@ -335,14 +353,10 @@ class FnoNet:
         x_in, x_out = self.xa, self.xb
         for l in range(L):
             Xs = _addr(self.Xs, l * m * m * C2 * B)
-            self._gemm(_addr(self.Fy), (0, H, 1), _addr(self.Z), (H * m2, m2, 1), _addr(self.Pm),
-                       (m2 * m2, m2, 1), m2, m2, H, batch=CB)
-            call("namsa_modes_combine", ptr(self.Pm), Xs, C, B, m, st)
+            self._y_forward(Xs, B)
             self._gemm(self._p("G", l), (C2 * C2, C2, 1), Xs, (C2 * B, B, 1), ptr(self.Ys), (C2 * B, B, 1),
                        C2, B, C2, batch=m * m)
-            call("namsa_modes_expand", ptr(self.Ys), ptr(self.E), C, B, m, st)
-            self._gemm(_addr(self.Fy), (0, 1, H), _addr(self.E), (m2 * m2, m2, 1), _addr(self.Zp),
-                       (H * m2, m2, 1), H, m2, m2, batch=CB)
+            self._spectral_rows(ptr(self.Ys), B)
             alpha = np.float32(1.0 / (H * W))
             if l < L - 1:
                 call("namsa_fno_layer", ptr(x_in), ptr(self.Zp), ptr(self.fx_bf), ptr(self.fxT_bf),
