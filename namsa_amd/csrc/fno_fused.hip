@@ -10,31 +10,27 @@
 //
 // with Fx[x][q] the truncated row DFT ([cos | -sin] of the m retained x modes,
 // 2m = 32 columns), Zp_l the row-inverse operand the small mode-space
-// products leave (mode mixing and the y transforms stay on the strided GEMM),
+// products leave (mode mixing, on the strided GEMM, and the y transforms),
 // and Z_{l+1} the next layer's row DFT.  One wavefront streams one row in
 // 32-pixel tiles: the first product is four v_mfma_f32_32x32x16_bf16 with
 // K = 32 modes + 32 channels (both operands read 16 bytes per lane straight
-// from memory), the tile goes through LDS once (bias, GELU, bf16) and leaves
-// as the next activation, and two more MFMAs fold it into the next row DFT.
+// from memory), the tile goes through LDS once (after bias and GELU, as bf16)
+// and leaves as the next activation, and two more MFMAs fold it into the next
+// row DFT.
 // Each layer therefore reads and writes the activation once: 128 bytes per
 // pixel.  The lift (features -> 32 channels) also forms layer 0's row DFT;
 // the last layer feeds the pointwise head (32 -> 64 -> 2) instead.
 //
-// MFMA 32x32x16 operand layout (lane l, 8 bf16 per operand register set):
-//   A: row l%32, k = 8*(l/32) + e      B: column l%32, k = 8*(l/32) + e
-//   D: 16 floats, register r holds row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 // Z / Zp rows are ordered (c, b, y): row (c * B + b) * H + y, 32 floats each,
 // the layout of the strided GEMM path's row-DFT output.
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
+#include "mfma.hpp"
 #include "namsa_hip.h"
 
 namespace namsa {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kCh = 32;        // channels
 constexpr int kQ = 32;         // 2m row-DFT columns
@@ -44,22 +40,16 @@ constexpr int kPitch = 40;     // LDS row pitch in bf16 (80 bytes: 16-byte align
 constexpr int kWaves = 4;
 
 // tanh-GELU, x/2 (1 + tanh(u)) = x (1 - 1 / (exp(2u) + 1)), u = sqrt(2/pi) (x + 0.044715 x^3);
-// the exponential form differs from tanhf by ~1e-7, far below the bf16 rounding of its result
+// the exponential form differs from tanhf by ~1e-7, far below the bf16 rounding of its result.
+// The quotient is one Newton step from the reciprocal's, which rounds as the
+// division does (the divisor lies in [1, 2^100], where its scaling steps have
+// nothing to do): 5 instructions for 11 of the 25.
 __device__ __forceinline__ float gelu_t(float x) {
   const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-  return x - x / (__expf(2.0f * u) + 1.0f);
+  const float d = fminf(__expf(2.0f * u) + 1.0f, 0x1p100f);
+  const float r = __builtin_amdgcn_rcpf(d), q = x * r;
+  return x - fmaf(fmaf(-d, q, x), r, q);
 }
-
-// The LDS tiles are private to a wavefront: its lanes exchange through them
-// in program order, so a wavefront-scope fence (no wait on other wavefronts)
-// is the only ordering the exchanges need.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ bf16x8 ld8(const __bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
 __device__ __forceinline__ bf16x8 cvt8(const float* p, float scale) {
   const float4 a = *reinterpret_cast<const float4*>(p);
@@ -76,232 +66,220 @@ __device__ __forceinline__ bf16x8 cvt8(const float* p, float scale) {
   return v;
 }
 
+// What the lanes of a wavefront exchange of a tile.
+struct alignas(16) Exchange {
+  __bf16 by_channel[kCh][kPitch], by_pixel[kTile][kPitch];
+};
+
 struct RowGeom {
   int rows, W, Wp, H, B;
 };
 
-// The row DFT of one 32-pixel tile held transposed in LDS (tt[c][x]) added to
-// zacc(q, c): A(q, k = x) = fxT[q][x0 + k], B(k = x, c) = tt[c][k].
-__device__ __forceinline__ void tile_row_dft(f32x16& zacc, const __bf16* __restrict__ fxT, int Wp, int x0,
-                                             const __bf16 (*tt)[kPitch], int lane) {
+// A tile's values, channel 8 (i / 4) + 4 half + i % 4 of pixel x0 + col in v[i],
+// leave rounded as the next activation and are added to the row's DFT:
+// zacc(c, q) += sum_x v(c, x) fxT[q][x], f holding the tile's rows of fxT.  Both
+// pass through LDS: for the DFT the pixels have to lie along k, and the
+// activation is stored in whole 1 KiB runs.  (A layer of 64 images of 170 x 170
+// took 107 us with 16 bytes of each 64 a store and Z in pieces of 16 bytes.)
+__device__ __forceinline__ void tile_out(const f32x16& v, f32x16& zacc, const bf16x8 (&f)[2], int x0, int W,
+                                         Exchange& ex, __bf16* __restrict__ row, int lane) {
+  const int col = lane & 31, half = lane >> 5, kh = 8 * half;
+  const bool in = x0 + col < W;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    const int k = 16 * s + 8 * (lane >> 5);
-    const bf16x8 a = ld8(fxT + static_cast<long long>(lane & 31) * Wp + x0 + k);
-    const bf16x8 b = ld8(&tt[lane & 31][k]);
-    zacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, zacc, 0, 0, 0);
+    bf16x8 h;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int i = 8 * s + e;
+      h[e] = __bf16(in ? v[i] : 0.0f);
+      ex.by_channel[8 * (i >> 2) + 4 * half + (i & 3)][col] = h[e];
+    }
+    *reinterpret_cast<bf16x8*>(&ex.by_pixel[col][16 * s + kh]) = rows_to_k(h);
   }
+  wave_sync();
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int px = 16 * s + (lane >> 2);
+    const bf16x8 h = ld8(&ex.by_pixel[px][8 * (lane & 3)]);
+    if (x0 + px < W) *reinterpret_cast<bf16x8*>(row + static_cast<long long>(x0 + px) * kCh + 8 * (lane & 3)) = h;
+    zacc = mfma(ld8(&ex.by_channel[col][16 * s + kh]), f[s], zacc);
+  }
+  wave_sync();
 }
 
+// Z's rows of the image row, whole rows of 32 q a store.
 __device__ __forceinline__ void store_z(float* __restrict__ Z, const f32x16& zacc, const RowGeom& g, int r,
                                         int lane) {
   const int b = r / g.H, y = r % g.H;
-  const int c = lane & 31;
-  float* zr = Z + ((static_cast<long long>(c) * g.B + b) * g.H + y) * kQ;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) zr[8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)] = zacc[i];
+  for (int i = 0; i < 16; ++i) {
+    const int c = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+    Z[((static_cast<long long>(c) * g.B + b) * g.H + y) * kQ + (lane & 31)] = zacc[i];
+  }
 }
 
 // x0 = Wl u + bl (u channel-major [cin][rows * W]) and layer 0's row DFT.
 // Per 32-pixel tile one MFMA with K = 16 (cin inputs, the rest zero):
-// A(x, k) = u[k][x], B(k, o) = Wl[o][k].
+// A(o, k) = Wl[o][k], B(k, x) = u[k][x], the next tile's read while one
+// computes.  Bound by the activation's writes and the wavefronts' serial tiles:
+// 64 images of 170 x 170 85 -> 43 us (the pixel in the lane throughout, no
+// branch around a load).
 __global__ void __launch_bounds__(256)
 fno_lift_kernel(const float* __restrict__ u, int cin, const float* __restrict__ Wl, const float* __restrict__ bl,
                 const __bf16* __restrict__ fxT, RowGeom g, __bf16* __restrict__ xout, float* __restrict__ Z) {
-  __shared__ __align__(16) __bf16 tt_all[kWaves][kCh][kPitch];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ Exchange exchange[kWaves];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = blockIdx.x * kWaves + wave;
-  const bool live = r < g.rows;
-  __bf16 (*tt)[kPitch] = tt_all[wave];
+  if (r >= g.rows) return;
   const long long n = static_cast<long long>(g.rows) * g.W;
-  const int col = lane & 31, kh = 8 * (lane >> 5);
-  bf16x8 wop;                                    // B(k = kh + e, o = col)
+  const int col = lane & 31, half = lane >> 5, kh = 8 * half;
+  bf16x8 wop;                                    // A(o = col, k = kh + e)
 #pragma unroll
-  for (int e = 0; e < 8; ++e) wop[e] = __bf16(kh + e < cin ? Wl[col * cin + kh + e] : 0.0f);
-  const float bo = bl[col];
-  f32x16 zacc;
+  for (int e = 0; e < 8; ++e) {
+    const float w = Wl[col * cin + min(kh + e, cin - 1)];
+    wop[e] = __bf16(kh + e < cin ? w : 0.0f);
+  }
+  float bias[16];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) zacc[i] = 0.0f;
+  for (int i = 0; i < 16; ++i) bias[i] = bl[8 * (i >> 2) + 4 * half + (i & 3)];
+  // input e at this lane's pixel; the upper half's inputs do not exist (cin <= 8), nor do pixels past the row
+  const float* ur = u + static_cast<long long>(r) * g.W;
+  auto load_in = [&](int px, float (&v)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = ur[min(e, cin - 1) * n + min(px, g.W - 1)];
+  };
+  const __bf16* fx_row = fxT + static_cast<long long>(col) * g.Wp + kh;
+  f32x16 zacc = zero16();
+  float next[8];
+  load_in(col, next);
   for (int x0 = 0; x0 < g.W; x0 += kTile) {
-    const int pa = x0 + col;                     // this lane's A row (pixel)
-    const bool va = live && pa < g.W;
     bf16x8 a;
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      a[e] = __bf16((va && kh + e < cin) ? u[(kh + e) * n + static_cast<long long>(r) * g.W + pa] : 0.0f);
-    f32x16 acc;
+    for (int e = 0; e < 8; ++e) a[e] = __bf16(kh + e < cin ? next[e] : 0.0f);
+    const bf16x8 f[2] = {ld8(fx_row + x0), ld8(fx_row + x0 + 16)};
+    load_in(x0 + kTile + col, next);
+    f32x16 acc = mfma(wop, a, zero16());
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wop, acc, 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int x = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-      tt[col][x] = __bf16(x0 + x < g.W ? acc[i] + bo : 0.0f);
-    }
-    wave_sync();
-    const int px = x0 + col;                     // store: lane -> pixel l%32, channels 16(l/32) .. +16
-    if (live && px < g.W) {
-      bf16x8 o0, o1;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        o0[e] = tt[16 * (lane >> 5) + e][col];
-        o1[e] = tt[16 * (lane >> 5) + 8 + e][col];
-      }
-      __bf16* dst = xout + (static_cast<long long>(r) * g.W + px) * kCh + 16 * (lane >> 5);
-      *reinterpret_cast<bf16x8*>(dst) = o0;
-      *reinterpret_cast<bf16x8*>(dst + 8) = o1;
-    }
-    tile_row_dft(zacc, fxT, g.Wp, x0, tt, lane);
-    wave_sync();
+    for (int i = 0; i < 16; ++i) acc[i] += bias[i];
+    tile_out(acc, zacc, f, x0, g.W, exchange[wave], xout + static_cast<long long>(r) * g.W * kCh, lane);
   }
-  if (live) store_z(Z, zacc, g, r, lane);
+  store_z(Z, zacc, g, r, lane);
 }
 
-// One Fourier layer.  last == 0: x_out = gelu(...) and Z_next; last == 1: no
+// One Fourier layer.  LAST == 0: x_out = gelu(...) and Z_next; LAST == 1: no
 // GELU, then the head out[t][p] = Q2 gelu(Q1 x + bq1) + bq2 (out channel-major
-// [2][rows * W] float).
+// [2][rows * W] float).  The pixel stays in the lane from the first product to
+// the last, so a product's result is the next one's operand after an exchange
+// between the wavefront's halves.  A layer is bound by its 326 MB (3.7 TB/s),
+// the head by the arithmetic of 64 GELUs a pixel.  64 images of 170 x 170: 110 -> 88 us, with
+// the head 182 -> 117, against the channel in the lane and each result passed
+// through LDS.
 template <int LAST>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 3)
 fno_layer_kernel(const __bf16* __restrict__ x_in, const float* __restrict__ Zp, const __bf16* __restrict__ fx,
                  const __bf16* __restrict__ fxT, const float* __restrict__ Wt, const float* __restrict__ bias,
                  float alpha, RowGeom g, __bf16* __restrict__ x_out, float* __restrict__ Z_next,
                  const float* __restrict__ Q1, const float* __restrict__ bq1, const float* __restrict__ Q2,
                  const float* __restrict__ bq2, float* __restrict__ out) {
-  __shared__ __align__(16) __bf16 tt_all[kWaves][kCh][kPitch];           // [c][x] (LAST: [x][c])
-  constexpr int kHPitch = kHid + 8;                                      // 144-byte rows: 16-byte aligned
-  __shared__ __align__(16) __bf16 hb_all[LAST ? kWaves : 1][LAST ? kTile : 1][LAST ? kHPitch : 8];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ Exchange exchange[LAST ? 1 : kWaves];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = blockIdx.x * kWaves + wave;
-  const bool live = r < g.rows;
-  const int rr = live ? r : 0;                  // masked waves read row 0 and write nothing
-  __bf16 (*tt)[kPitch] = tt_all[wave];
-  const int b = rr / g.H, y = rr % g.H;
-  const int col = lane & 31, kh = 8 * (lane >> 5);
+  if (r >= g.rows) return;
+  const int b = r / g.H, y = r % g.H;
+  const int col = lane & 31, half = lane >> 5, kh = 8 * half;
 
-  // B operands of the layer product, the same for every tile of the row:
-  // k < 32: alpha Zp[o][q] (q = k), k >= 32: W[o][c] (c = k - 32), o = column
-  bf16x8 bop[4];
+  // A operands of the layer product, the same for every tile of the row:
+  // k < 32: alpha Zp[o][q] (q = k), k >= 32: W[o][c] (c = k - 32), o = col
+  bf16x8 aop[4];
   const float* zp_row = Zp + ((static_cast<long long>(col) * g.B + b) * g.H + y) * kQ;
-  bop[0] = cvt8(zp_row + kh, alpha);
-  bop[1] = cvt8(zp_row + 16 + kh, alpha);
-  bop[2] = cvt8(Wt + col * kCh + kh, 1.0f);
-  bop[3] = cvt8(Wt + col * kCh + 16 + kh, 1.0f);
-  const float bo = bias[col];
-  bf16x8 q1op[2][2];                            // head operands B(k = c, j) = Q1[j][c], constant per wave
-  bf16x8 q2op[4];                               // B(k = j, t) = Q2[t][j] for t = col < 2, else 0
+  aop[0] = cvt8(zp_row + kh, alpha);
+  aop[1] = cvt8(zp_row + 16 + kh, alpha);
+  aop[2] = cvt8(Wt + col * kCh + kh, 1.0f);
+  aop[3] = cvt8(Wt + col * kCh + 16 + kh, 1.0f);
+  float bo[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) bo[i] = bias[8 * (i >> 2) + 4 * half + (i & 3)];
+  bf16x8 q1op[2][2];                            // head operands A(j, k = c) = Q1[j][c], constant per wave
+  bf16x8 q2op[4];                               // A(t, k = j) = Q2[t][j] for t = col < 2, else 0
+  float b1[LAST ? 2 : 1][16];
   if (LAST) {
 #pragma unroll
-    for (int jb = 0; jb < 2; ++jb)
+    for (int jb = 0; jb < 2; ++jb) {
 #pragma unroll
       for (int s = 0; s < 2; ++s) q1op[jb][s] = cvt8(Q1 + (32 * jb + col) * kCh + 16 * s + kh, 1.0f);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) b1[jb][i] = bq1[32 * jb + 8 * (i >> 2) + 4 * half + (i & 3)];
+    }
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
       for (int e = 0; e < 8; ++e) q2op[s][e] = __bf16(col < 2 ? Q2[col * kHid + 16 * s + kh + e] : 0.0f);
   }
 
-  f32x16 zacc;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) zacc[i] = 0.0f;
+  f32x16 zacc = zero16();
   const long long n = static_cast<long long>(g.rows) * g.W;
-  // channel operands A(x, k = 32 + 16 s + kh ..) of a tile; the next tile's are loaded while this one computes
-  auto load_ch = [&](int x0, bf16x8 (&a)[2]) {
-    const int pa = x0 + col;
+  // a tile's operands, modes B(k = 16 s + kh .., x) and channels B(k = 32 + 16 s
+  // + kh .., x), are loaded while the tile before computes; pixels past the row
+  // read its last one, their results go nowhere
+  const __bf16* x_row = x_in + static_cast<long long>(r) * g.W * kCh + kh;
+  const __bf16* fx_row = fxT + static_cast<long long>(col) * g.Wp + kh;
+  auto load = [&](int x0, bf16x8 (&a)[4]) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      if (pa < g.W) {
-        a[s] = ld8(x_in + (static_cast<long long>(rr) * g.W + pa) * kCh + 16 * s + kh);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) a[s][e] = __bf16(0.0f);
-      }
+      a[s] = ld8(fx + static_cast<long long>(min(x0 + col, g.Wp - 1)) * kQ + 16 * s + kh);
+      a[2 + s] = ld8(x_row + static_cast<long long>(min(x0 + col, g.W - 1)) * kCh + 16 * s);
     }
   };
-  bf16x8 anext[2];
-  load_ch(0, anext);
+  bf16x8 next[4];
+  load(0, next);
   for (int x0 = 0; x0 < g.W; x0 += kTile) {
-    const int pa = x0 + col;                    // this lane's A row (pixel)
-    bf16x8 ach[2] = {anext[0], anext[1]};
-    if (x0 + kTile < g.W) load_ch(x0 + kTile, anext);
-    f32x16 acc;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {               // k = 16 s + kh .. : modes
-      const bf16x8 a = ld8(fx + static_cast<long long>(pa) * kQ + 16 * s + kh);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bop[s], acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int s = 0; s < 2; ++s)                 // k = 32 + 16 s + kh .. : channels
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ach[s], bop[2 + s], acc, 0, 0, 0);
-    // epilogue: pixel x = 8(i/4) + 4(l/32) + i%4 of the tile, channel o = col
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int x = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-      float v = acc[i] + bo;
-      if (!LAST) v = gelu_t(v);
-      if (x0 + x >= g.W) v = 0.0f;
-      if (LAST) tt[x][col] = __bf16(v);
-      else tt[col][x] = __bf16(v);
-    }
-    wave_sync();
+    const int px = x0 + col;                    // this lane's pixel
+    const bf16x8 bop[4] = {next[0], next[1], next[2], next[3]};
+    bf16x8 f[2];                                // asked for before the next tile: a wait for it is none for that
     if constexpr (!LAST) {
-      // the tile leaves as the next activation: lane -> pixel l%32, channels 16(l/32) .. +16
-      const int px = x0 + col;
-      if (live && px < g.W) {
-        bf16x8 o0, o1;
+      f[0] = ld8(fx_row + x0);
+      f[1] = ld8(fx_row + x0 + 16);
+    }
+    load(x0 + kTile, next);
+    f32x16 acc = zero16();
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          o0[j] = tt[16 * (lane >> 5) + j][col];
-          o1[j] = tt[16 * (lane >> 5) + 8 + j][col];
-        }
-        __bf16* dst = x_out + (static_cast<long long>(r) * g.W + px) * kCh + 16 * (lane >> 5);
-        *reinterpret_cast<bf16x8*>(dst) = o0;
-        *reinterpret_cast<bf16x8*>(dst + 8) = o1;
-      }
-      tile_row_dft(zacc, fxT, g.Wp, x0, tt, lane);
+    for (int s = 0; s < 4; ++s) acc = mfma(aop[s], bop[s], acc);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] += bo[i];
+    if constexpr (!LAST) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] = gelu_t(acc[i]);
+      tile_out(acc, zacc, f, x0, g.W, exchange[wave], x_out + static_cast<long long>(r) * g.W * kCh, lane);
     } else {
-      // head: h = gelu(Q1 x + bq1) as two 32-wide MFMA blocks, A(x, k = c) = tt[x][c], kept bf16 in LDS
-      __bf16 (*hb)[kHPitch] = hb_all[wave];
+      // head: h = gelu(Q1 x + bq1) as two 32-row blocks, out[t] = Q2[t] . h + bq2[t] over K = 64
+      bf16x8 xb[2];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xb[s][e] = __bf16(acc[8 * s + e]);
+        xb[s] = rows_to_k(xb[s]);
+      }
+      f32x16 oacc = zero16();
 #pragma unroll
       for (int jb = 0; jb < 2; ++jb) {
-        f32x16 hacc;
+        f32x16 hacc = zero16();
 #pragma unroll
-        for (int i = 0; i < 16; ++i) hacc[i] = 0.0f;
+        for (int s = 0; s < 2; ++s) hacc = mfma(q1op[jb][s], xb[s], hacc);
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-          const bf16x8 a = ld8(&tt[col][16 * s + kh]);
-          hacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, q1op[jb][s], hacc, 0, 0, 0);
+          bf16x8 h;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) h[e] = __bf16(gelu_t(hacc[8 * s + e] + b1[jb][8 * s + e]));
+          oacc = mfma(q2op[2 * jb + s], rows_to_k(h), oacc);
         }
-        const float bj = bq1[32 * jb + col];
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          hb[8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)][32 * jb + col] = __bf16(gelu_t(hacc[i] + bj));
       }
-      wave_sync();
-      // out[t][p] = Q2[t] . h + bq2[t]: four MFMAs with K = 64, A(x, k = j) = hb[x][j]; columns t < 2 kept
-      f32x16 oacc;
+      if (half == 0 && px < g.W) {              // rows t < 2 of the result
 #pragma unroll
-      for (int i = 0; i < 16; ++i) oacc[i] = 0.0f;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const bf16x8 a = ld8(&hb[col][16 * s + kh]);
-        oacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, q2op[s], oacc, 0, 0, 0);
-      }
-      if (live && col < 2) {
-        const float bt = bq2[col];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int px = x0 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-          if (px < g.W) out[col * n + static_cast<long long>(r) * g.W + px] = oacc[i] + bt;
-        }
+        for (int t = 0; t < 2; ++t) out[t * n + static_cast<long long>(r) * g.W + px] = oacc[t] + bq2[t];
       }
     }
-    wave_sync();
   }
-  if constexpr (!LAST) {
-    if (live) store_z(Z_next, zacc, g, r, lane);
-  }
+  if constexpr (!LAST) store_z(Z_next, zacc, g, r, lane);
 }
 
 int check_geom(int B, int H, int W, int Wp, const char* who) {

@@ -8,33 +8,23 @@
 //   inverse:  E[0p][0q] = E[1p][1q] = Yr_pq, E[0p][1q] = -E[1p][0q] = Yi_pq,
 //             Zp[y][(t,q)] = sum_(r,p) Fy[(r,p)][y] E[(r,p)][(t,q)]
 //
-// One workgroup for a channel of a sample.  MFMA 32x32x16 operand layout (lane
-// l, 8 bf16 per operand register set):
-//   A: row l%32, k = 8*(l/32) + e      B: column l%32, k = 8*(l/32) + e
-//   D: 16 floats, register r holds row 8*(r/4) + 4*(l/32) + r%4, column l%32.
+// One workgroup for a channel of a sample.
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
+#include "mfma.hpp"
 #include "namsa_hip.h"
 
 namespace namsa {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-
 constexpr int kM = 16;                  // modes an axis
 constexpr int kM2 = 2 * kM;
 constexpr int kSteps = 3;               // steps of 16 y a wavefront has in flight
-constexpr int kRawBuffer = 0x00020000;  // gfx9 raw-buffer resource word 3
-
-__device__ __forceinline__ bf16x8 ld8(const __bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
 // Reads past the H rows of this channel and sample give 0, stores there are dropped.
 __device__ __forceinline__ Rsrc rows_of(const float* Z, int cb, int H) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Z) + static_cast<long long>(cb) * H * kM2, 0,
-                                           4 * kM2 * H, kRawBuffer);
+  return buffer_of(Z + static_cast<long long>(cb) * H * kM2, 4 * kM2 * H);
 }
 
 // Bound by reading Z once.  The four wavefronts take every fourth step of 16 y,
@@ -49,17 +39,14 @@ __global__ void __launch_bounds__(256) modes_forward_kernel(const float* __restr
   const int col = lane & 31, half = lane >> 5, kh = 8 * half;
   const int cb = blockIdx.x, c = cb / B, b = cb % B;
   const Rsrc rz = rows_of(Z, cb, H);
-  f32x16 acc;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+  f32x16 acc = zero16();
   for (int k0 = 16 * wave; k0 < H; k0 += 64 * kSteps) {
     float z[kSteps][8];
 #pragma unroll
     for (int s = 0; s < kSteps; ++s)
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        z[s][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rz, 4 * (kM2 * kh + col),
-                                                                                 4 * kM2 * (k0 + 64 * s + e), 0));
+        z[s][e] = load_b32(rz, 4 * (kM2 * kh + col), 4 * kM2 * (k0 + 64 * s + e));
     bf16x8 a[kSteps];
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) a[s] = ld8(fy + col * Hp + min(k0 + 64 * s, Hp - 16) + kh);
@@ -69,7 +56,7 @@ __global__ void __launch_bounds__(256) modes_forward_kernel(const float* __restr
       bf16x8 v;
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = __bf16(z[s][e]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], v, acc, 0, 0, 0);
+      acc = mfma(a[s], v, acc);
     }
   }
   if (wave > 0) {
@@ -118,17 +105,11 @@ __global__ void __launch_bounds__(256) modes_inverse_kernel(const float* __restr
   const bf16x8 e0 = ld8(&E[col][kh]), e1 = ld8(&E[col][16 + kh]);
   for (int y0 = 32 * wave; y0 < H; y0 += 128) {
     const __bf16* f = fyT + (y0 + col) * kM2 + kh;
-    f32x16 acc;
+    f32x16 acc = mfma(ld8(f), e0, zero16());
+    acc = mfma(ld8(f + 16), e1, acc);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(f), e0, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(f + 16), e1, acc, 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float v = acc[i];
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rz, 4 * (4 * kM2 * half + col),
-                                            4 * kM2 * (y0 + 8 * (i >> 2) + (i & 3)), 0);
-    }
+    for (int i = 0; i < 16; ++i)
+      store_b32(acc[i], rz, 4 * (4 * kM2 * half + col), 4 * kM2 * (y0 + 8 * (i >> 2) + (i & 3)));
   }
 }
 

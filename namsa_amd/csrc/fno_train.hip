@@ -12,9 +12,6 @@
 // previous one's gradient, starts from).  The small mode-space products
 // between Z and Zp stay on the strided GEMM.
 //
-// MFMA 32x32x16 operand layout (lane l, 8 bf16 per operand register set):
-//   A: row l%32, k = 8*(l/32) + e      B: column l%32, k = 8*(l/32) + e
-//   D: 16 floats, register r holds row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 // Z / Zp rows are ordered (c, b, y): row (c * B + b) * H + y, 32 floats each.
 #include <hip/hip_runtime.h>
 
@@ -22,13 +19,11 @@
 
 #include "common.hpp"
 #include "gelu.hpp"
+#include "mfma.hpp"
 #include "namsa_hip.h"
 
 namespace namsa {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kCh = 32;                 // channels
 constexpr int kQ = 32;                  // 2m row-DFT columns
@@ -37,52 +32,6 @@ constexpr int kPitch = 40;              // LDS row pitch in bf16 (80 bytes: 16-b
 constexpr int kTiles = 2;               // tiles of a wavefront
 constexpr int kRunTiles = 12;           // tiles of a workgroup at a time
 constexpr int kTileBytes = 2 * kCh * kPitch + 2 * kQ * kTile;  // a rounded tile and its row-DFT operand
-constexpr int kRawBuffer = 0x00020000;  // gfx9 raw-buffer resource word 3
-constexpr int kNowhere = 0x7ffffffc;    // a byte offset past every buffer: stores there are dropped
-
-__device__ __forceinline__ bf16x8 ld8(const __bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
-
-// A wavefront exchanges through its own LDS tile in program order: only the
-// compiler has to be held to it.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-
-// Accesses through a buffer resource at a lane's and a scalar byte offset;
-// reads past its end give 0, stores there are dropped.
-__device__ __forceinline__ float load_b32(Rsrc r, int lane_at, int at) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, lane_at, at, 0));
-}
-__device__ __forceinline__ void store_b32(float v, Rsrc r, int lane_at, int at) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, lane_at, at, 0);
-}
-__device__ __forceinline__ bf16x8 load_bf8(Rsrc r, int lane_at, int at) {
-  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, lane_at, at, 0));
-}
-// eight consecutive floats, rounded to bf16
-__device__ __forceinline__ bf16x8 load_f8(Rsrc r, int lane_at, int at) {
-  const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, lane_at, at, 0);
-  const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(r, lane_at, at + 16, 0);
-  bf16x8 v;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    v[e] = __bf16(__builtin_bit_cast(float, static_cast<unsigned>(a[e])));
-    v[e + 4] = __bf16(__builtin_bit_cast(float, static_cast<unsigned>(b[e])));
-  }
-  return v;
-}
-
-__device__ __forceinline__ f32x16 zero16() {
-  f32x16 v;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) v[i] = 0.0f;
-  return v;
-}
 
 // v + alpha x with the product rounded first, as the separate products do
 __device__ __forceinline__ float add_scaled(float v, float alpha, float x) {
@@ -140,16 +89,11 @@ __global__ void __launch_bounds__(64 * kRunTiles / kTiles, 2) fno_rows_kernel(Ro
   const int col = lane & 31, half = lane >> 5, kh = 8 * half;
   const int b = r / g.H, y = r % g.H;
   const int zrow = 4 * kQ * ((col * g.B + b) * g.H + y);  // byte offset of channel `col` in Z and Zp
-  const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(g.x), 0, g.cin * g.pitch, kRawBuffer);
-  const auto ro = __builtin_amdgcn_make_buffer_rsrc(g.out, 0, kCh * g.pitch, kRawBuffer);
-  const auto rp = __builtin_amdgcn_make_buffer_rsrc(ACT == kGelu ? g.pre_out : const_cast<float*>(g.pre_in), 0,
-                                                    ACT == kPlain ? 0 : kCh * g.pitch, kRawBuffer);
-  const auto rz = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(g.Zp), 0, MODES ? 4 * kQ * kCh * g.rows : 0,
-                                                    kRawBuffer);
-  const auto rf = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(g.fx), 0, MODES ? 2 * kQ * g.Wp : 0, kRawBuffer);
-  const auto rt = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(g.fxT), 0, DFT ? 2 * kQ * g.Wp : 0, kRawBuffer);
-  const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(g.Wt), 0, 4 * kCh * g.cin, kRawBuffer);
-  const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(g.bias), 0, BIAS ? 4 * kCh : 0, kRawBuffer);
+  const Rsrc rx = buffer_of(g.x, g.cin * g.pitch), ro = buffer_of(g.out, kCh * g.pitch);
+  const Rsrc rp = buffer_of(ACT == kGelu ? g.pre_out : g.pre_in, ACT == kPlain ? 0 : kCh * g.pitch);
+  const Rsrc rz = buffer_of(g.Zp, MODES ? 4 * kQ * kCh * g.rows : 0);
+  const Rsrc rf = buffer_of(g.fx, MODES ? 2 * kQ * g.Wp : 0), rt = buffer_of(g.fxT, DFT ? 2 * kQ * g.Wp : 0);
+  const Rsrc rw = buffer_of(g.Wt, 4 * kCh * g.cin), rb = buffer_of(g.bias, BIAS ? 4 * kCh : 0);
   const int row = 4 * r * g.W;  // byte offset of the image row in a channel
 
   f32x16 zacc = zero16();
@@ -213,15 +157,14 @@ __global__ void __launch_bounds__(64 * kRunTiles / kTiles, 2) fno_rows_kernel(Ro
       if constexpr (MODES) {
 #pragma unroll
         for (int s = 0; s < 2; ++s)
-          modes = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[s], load_bf8(rf, 2 * (px * kQ + kh), 32 * s), modes, 0, 0,
-                                                          0);
+          modes = mfma(am[s], load_bf8(rf, 2 * (px * kQ + kh), 32 * s), modes);
       }
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         bf16x8 c;
 #pragma unroll
         for (int e = 0; e < 8; ++e) c[e] = __bf16(in[t][s][e]);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aw[s], c, acc, 0, 0, 0);
+        acc = mfma(aw[s], c, acc);
       }
       const int at = px < g.W ? 4 * half * g.pitch + 4 * px : kNowhere;
 #pragma unroll
@@ -249,7 +192,7 @@ __global__ void __launch_bounds__(64 * kRunTiles / kTiles, 2) fno_rows_kernel(Ro
           const bf16x8* f = reinterpret_cast<const bf16x8*>(t + kCh * kPitch * 2);
 #pragma unroll
           for (int s = 0; s < 2; ++s)
-            zacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[64 * s + lane], ld8(&zt[col][16 * s + kh]), zacc, 0, 0, 0);
+            zacc = mfma(f[64 * s + lane], ld8(&zt[col][16 * s + kh]), zacc);
         }
       }
       if (32 * (t0 + kTiles * waves) < g.W) __syncthreads();
@@ -301,10 +244,6 @@ struct HeadArgs {
   const float* gout;                      // [2][n]
   float *gx, *gQ1, *gbq1, *gQ2, *gbq2;
 };
-
-__device__ __forceinline__ Rsrc buffer_of(const void* p, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, kRawBuffer);
-}
 
 // 16 channels' steps of a tile, channels 16 s + 8 half + e at this lane's pixel
 __device__ __forceinline__ void load_pixels(float (&v)[2][8], Rsrc r, int pitch, int px, int n, int kh) {
@@ -358,20 +297,13 @@ __global__ void __launch_bounds__(256) fno_head_kernel(HeadArgs g) {
     for (int jb = 0; jb < 2; ++jb) {
       f32x16 acc = zero16();
 #pragma unroll
-      for (int s = 0; s < 2; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q1[jb][s], bx[s], acc, 0, 0, 0);
+      for (int s = 0; s < 2; ++s) acc = mfma(q1[jb][s], bx[s], acc);
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        bf16x8 h;  // units 16 s + (0..3, 8..11 in the lower half; 4..7, 12..15 in the upper)
+        bf16x8 h;
 #pragma unroll
         for (int e = 0; e < 8; ++e) h[e] = __bf16(gelu_tanh(acc[8 * s + e] + b1[jb][8 * s + e]));
-        u32x4 w = __builtin_bit_cast(u32x4, h);
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const auto p = __builtin_amdgcn_permlane32_swap(w[e], w[e + 2], false, false);
-          w[e] = p[0];
-          w[e + 2] = p[1];
-        }
-        out = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q2[2 * jb + s], __builtin_bit_cast(bf16x8, w), out, 0, 0, 0);
+        out = mfma(q2[2 * jb + s], rows_to_k(h), out);
       }
     }
 #pragma unroll
@@ -460,29 +392,29 @@ __global__ void __launch_bounds__(64 * kHeadWaves, 2) fno_head_backward_kernel(H
     for (int jb = 0; jb < 2; ++jb) {
       f32x16 pre = zero16();
 #pragma unroll
-      for (int s = 0; s < 2; ++s) pre = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bx[s], q1[jb][s], pre, 0, 0, 0);
-      const f32x16 gh0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(go, q2[jb], zero16(), 0, 0, 0);
+      for (int s = 0; s < 2; ++s) pre = mfma(bx[s], q1[jb][s], pre);
+      const f32x16 gh0 = mfma(go, q2[jb], zero16());
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         bf16x8 h, gh;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int i = 8 * s + e;
-          const float v = pre[i] + b1[jb], t = gelu_t(v);
+          const float v = pre[i] + b1[jb], t = gelu_inner(v);
           h[e] = __bf16(gelu_tanh(v, t));
           gh[e] = __bf16(gh0[i] * gelu_grad_tanh(v, t));
           tt[8 * (i >> 2) + 4 * half + (i & 3)][32 * jb + col] = gh[e];
         }
-        gq1[jb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gh, xt[s], gq1[jb], 0, 0, 0);
-        gq2[jb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gt[s], h, gq2[jb], 0, 0, 0);
-        gq2[jb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, gh, gq2[jb], 0, 0, 0);
+        gq1[jb] = mfma(gh, xt[s], gq1[jb]);
+        gq2[jb] = mfma(gt[s], h, gq2[jb]);
+        gq2[jb] = mfma(ones, gh, gq2[jb]);
       }
     }
     wave_sync();
     f32x16 gx = zero16();
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      gx = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q1t[s], ld8(&tt[col][16 * s + kh]), gx, 0, 0, 0);
+      gx = mfma(q1t[s], ld8(&tt[col][16 * s + kh]), gx);
     wave_sync();
     const int at = px < g.n ? 4 * half * pitch + 4 * px : kNowhere;
 #pragma unroll
