@@ -86,6 +86,18 @@ int namsa_atomic_tables(const double* params, int nZ, int Py, int Px, double ran
                         int oversample, float* tables, void* stream);
 
 /*
+ * Sites grouped by slice for the builders below (replaces the masks of
+ * namsa/msa.py:584-604): slice s holds bounds[s] <= z < bounds[s+1], sites keep
+ * their input order, sites outside every slice are left out.
+ *   xyz: [A][3] float32, z: [A] its third column, Z: [A] atomic numbers
+ *   unique_Z: [nZ] sorted, bounds: [S+1] nondecreasing; py, px: pixel sizes
+ *   sites: room for [A][3] int32 (index in unique_Z, int(y/py), int(x/px))
+ *   offsets: [S+1] int32
+ */
+int namsa_bin_sites(const float* xyz, const float* z, const long long* Z, int A, const long long* unique_Z, int nZ,
+                    const float* bounds, int S, double py, double px, int* sites, int* offsets, void* stream);
+
+/*
  * Transmission slices t = exp(i sigma V) (replaces BuildScatteringPotential,
  * namsa/potential_kernels.cu:5-60, launched at namsa/msa.py:626-639).
  *   tables:        [nZ][Py][Px] float32

@@ -34,6 +34,7 @@ SIGNATURES = {
     "namsa_init": (_i, [_i]),
     "namsa_fft_supported": (_i, [_i]),
     "namsa_atomic_tables": (_i, [_vp, _i, _i, _i, _d, _i, _vp, _vp]),
+    "namsa_bin_sites": (_i, [_vp, _vp, _vp, _i, _vp, _i, _vp, _i, _d, _d, _vp, _vp, _vp]),
     "namsa_build_slices": (_i, [_vp, _i, _i, _i, _vp, _vp, _i, _i, _i, _f, _vp, _vp]),
     "namsa_probe_k": (_i, [_i, _i, _f, _f, _f, _f, _f, _f, _i, _f, _vp, _vp, _vp]),
     "namsa_propagator": (_i, [_i, _i, _f, _f, _f, _f, _vp, _vp, _vp]),

@@ -15,6 +15,8 @@
 // ballot compaction) only those whose clipped footprint overlaps the tile, and accumulates table
 // values for its pixels in float32 in site order; exp(i sigma V) with the NaN
 // guard of potential_kernels.cu:48-57 is fused into the store.
+#include <climits>
+
 #include "common.hpp"
 #include "namsa_hip.h"
 
@@ -440,6 +442,97 @@ __global__ void __launch_bounds__(256) integrate_slices_kernel(const double* pot
   }
 }
 
+// Sites of one slice per workgroup, in input order: every workgroup reads all
+// depths (16 bytes a thread, from the L2 caches after the first), first to
+// count the sites before its slice, then to place its own, ranked by ballot
+// within a wavefront and by a running sum over wavefronts.  The reads grow with
+// S times A, but a workgroup's chain of steps only with A, and no list of a
+// site per step and slice has to be kept: 73,000 sites in 150 slices take
+// 73 us, 2.4 million in 310 3.6 ms, where the host's sorted lookup, stable
+// sort and three gathers took 7.3 and 350 ms.
+constexpr int kBinThreads = 1024;
+
+// truncation as the host's conversion has it: INT_MIN for what an int cannot hold
+__device__ __forceinline__ int to_int(double v) {
+  return v > -2147483649.0 && v < 2147483648.0 ? static_cast<int>(v) : INT_MIN;
+}
+
+__global__ void __launch_bounds__(kBinThreads)
+bin_sites_kernel(const float* __restrict__ xyz, const float* __restrict__ z, const long long* __restrict__ Z, int A,
+                 const long long* __restrict__ unique_Z, int nZ, const float* __restrict__ bounds, int S, double py,
+                 double px, int* __restrict__ sites, int* __restrict__ offsets) {
+  __shared__ int part[2][kBinThreads / 64];
+  const int s = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const float first = bounds[0], lo = bounds[s], hi = bounds[s + 1];
+  const int steps = (A + 4 * kBinThreads - 1) / (4 * kBinThreads);
+  auto load = [&](int step, float (&v)[4]) {  // NaN past the end: in no slice
+    const int i = 4 * (step * kBinThreads + static_cast<int>(threadIdx.x));
+    if (i + 3 < A) {
+      const float4 f = *reinterpret_cast<const float4*>(z + i);
+      v[0] = f.x;
+      v[1] = f.y;
+      v[2] = f.z;
+      v[3] = f.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = i + e < A ? z[i + e] : __builtin_nanf("");
+    }
+  };
+  int before = 0;
+  for (int step = 0; step < steps; ++step) {
+    float v[4];
+    load(step, v);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) before += (v[e] >= first) & (v[e] < lo);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
+  if (lane == 0) part[0][wave] = before;
+  __syncthreads();
+  int base = 0;
+  for (int w = 0; w < kBinThreads / 64; ++w) base += part[0][w];
+  if (threadIdx.x == 0) offsets[s] = base;
+  for (int step = 0; step < steps; ++step) {
+    float v[4];
+    load(step, v);
+    int mine = 0, rank = 0, all = 0;
+    const unsigned long long below = (1ull << lane) - 1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = (v[e] >= lo) & (v[e] < hi);
+      const unsigned long long m = __ballot(in);
+      mine |= in << e;
+      rank += __popcll(m & below);
+      all += __popcll(m);
+    }
+    int* sums = part[(step & 1) ^ 1];  // the other half may still be read
+    if (lane == 0) sums[wave] = all;
+    __syncthreads();
+    int total = 0;
+    for (int w = 0; w < kBinThreads / 64; ++w) {
+      if (w == wave) rank += total;
+      total += sums[w];
+    }
+    for (int e = 0; e < 4; ++e) {
+      if (!(mine >> e & 1)) continue;
+      const long long i = 4ll * (static_cast<long long>(step) * kBinThreads + threadIdx.x) + e;
+      int a = 0, b = nZ;  // the first element not below this site's
+      const long long own = Z[i];
+      while (a < b) {
+        const int mid = (a + b) >> 1;
+        if (unique_Z[mid] < own) a = mid + 1;
+        else b = mid;
+      }
+      int* out = sites + 3ll * (base + rank++);
+      out[0] = a;
+      out[1] = to_int(static_cast<double>(xyz[3 * i + 1]) / py);
+      out[2] = to_int(static_cast<double>(xyz[3 * i]) / px);
+    }
+    base += total;
+  }
+  if (s == S - 1 && threadIdx.x == 0) offsets[S] = base;
+}
+
 }  // namespace namsa
 
 using namespace namsa;
@@ -482,6 +575,15 @@ int namsa_atomic_tables(const double* params, int nZ, int Py, int Px, double ran
   hipLaunchKernelGGL(table_check_kernel, dim3(nZ), dim3(kTableThreads), 0, st, params, Py, Px, oversample, range,
                      split ? 0 : 1, tables);
   return check_hip(hipGetLastError(), "atomic_tables_kernel launch");
+}
+
+int namsa_bin_sites(const float* xyz, const float* z, const long long* Z, int A, const long long* unique_Z, int nZ,
+                    const float* bounds, int S, double py, double px, int* sites, int* offsets, void* stream) {
+  if (!xyz || !z || !Z || !unique_Z || !bounds || !sites || !offsets || A <= 0 || A > (1 << 30) || nZ <= 0 || S <= 0)
+    return fail(kErrArg, "namsa_bin_sites: null argument or A=%d nZ=%d S=%d out of range", A, nZ, S);
+  hipLaunchKernelGGL(bin_sites_kernel, dim3(S), dim3(kBinThreads), 0, as_stream(stream), xyz, z, Z, A, unique_Z, nZ,
+                     bounds, S, py, px, sites, offsets);
+  return check_hip(hipGetLastError(), "bin_sites_kernel launch");
 }
 
 int namsa_build_slices(const float* tables, int nZ, int Py, int Px, const int* sites,

@@ -298,6 +298,11 @@ class MSAGPU:
         host = self.tables_device.cpu().numpy()
         self.cached_pots = {int(Z): host[i] for i, Z in enumerate(self.unique_Z)}
 
+    def _slice_bounds(self, slice_thickness):
+        """(S, the S + 1 slice bounds as float32)."""
+        S = int(np.floor(np.float64(self.dims[-1]) / slice_thickness))
+        return S, np.array([n * slice_thickness for n in range(S + 1)], dtype=np.float64).astype(np.float32)
+
     def site_table(self, slice_thickness):
         """Sites grouped by slice under the MSAGPU rule (msa.py:584-604).
 
@@ -305,9 +310,8 @@ class MSAGPU:
         offsets int32 [S+1]).  Slice n holds float32(n dz) <= z < float32((n+1) dz);
         sites keep their input order inside a slice.
         """
-        S = int(np.floor(np.float64(self.dims[-1]) / slice_thickness))
+        S, bounds = self._slice_bounds(slice_thickness)
         z = self.supercell_xyz[:, 2]
-        bounds = np.array([n * slice_thickness for n in range(S + 1)], dtype=np.float64).astype(np.float32)
         sl = np.searchsorted(bounds, z, side="right") - 1
         keep = np.nonzero((sl >= 0) & (sl < S))[0]
         order = keep[np.argsort(sl[keep], kind="stable")]
@@ -319,6 +323,27 @@ class MSAGPU:
         offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
         return sites, offsets
 
+    def _sites_device(self, slice_thickness):
+        """``site_table`` in device memory (sites with room for every atom), binned there."""
+        torch = _torch()
+        dev = self._dev()
+        xyz, Z = self.supercell_xyz, self.supercell_Z
+        S, bounds = self._slice_bounds(slice_thickness)
+        if not (0 < S < 65536 and 0 < len(xyz) <= 1 << 30 and xyz.dtype == np.float32 and xyz.shape[1:] == (3,)
+                and Z.dtype == np.int64 and self.unique_Z.dtype == np.int64 and len(Z) == len(xyz)):
+            sites, offsets = self.site_table(slice_thickness)
+            return (torch.from_numpy(sites.reshape(-1)).to(dev) if len(sites) else None,
+                    torch.from_numpy(offsets).to(dev))
+        xyz_d = torch.from_numpy(np.ascontiguousarray(xyz)).to(dev)
+        z_d = xyz_d[:, 2].contiguous()
+        Z_d, unique_d, bounds_d = (torch.from_numpy(np.ascontiguousarray(a)).to(dev) for a in (Z, self.unique_Z, bounds))
+        sites = torch.empty(3 * len(xyz), dtype=torch.int32, device=dev)
+        offsets = torch.empty(S + 1, dtype=torch.int32, device=dev)
+        call("namsa_bin_sites", ptr(xyz_d), ptr(z_d), ptr(Z_d), len(xyz), ptr(unique_d), len(self.unique_Z),
+             ptr(bounds_d), S, float(self.pix_size[0]), float(self.pix_size[1]), ptr(sites), ptr(offsets),
+             stream_handle())
+        return sites, offsets
+
     def build_potential_slices(self, slice_thickness):
         """Transmission slices exp(i sigma V) on the GPU (msa.py:580-647)."""
         torch = _torch()
@@ -326,12 +351,10 @@ class MSAGPU:
         if not hasattr(self, "tables_device"):
             self.calc_atomic_potentials()
         self.slice_t = float(slice_thickness)
-        sites, offsets = self.site_table(slice_thickness)
-        self.num_slices = np.int32(len(offsets) - 1)
+        sites_d, offs_d = self._sites_device(slice_thickness)
+        self.num_slices = np.int32(len(offs_d) - 1)
         Ny, Nx = self._grid
         Py, Px = self.table_shape
-        sites_d = torch.from_numpy(sites.reshape(-1)).to(dev) if len(sites) else None
-        offs_d = torch.from_numpy(offsets).to(dev)
         self._t = torch.empty((int(self.num_slices), Ny, Nx), dtype=torch.complex64, device=dev)
         call("namsa_build_slices", ptr(self.tables_device), len(self.unique_Z), Py, Px,
              ptr(sites_d), ptr(offs_d), int(self.num_slices), Ny, Nx, np.float32(self.sigma),
