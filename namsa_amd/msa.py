@@ -183,8 +183,8 @@ class MSAGPU:
         arr = self._load_supercell(supercell)
         self.supercell_xyz = np.column_stack([arr["x"], arr["y"], arr["z"]]).astype(np.float32)
         self.supercell_Z = np.asarray(arr["atomic_number"]).astype(np.int64)
-        self.supercell_dw = np.asarray(arr["DW"], dtype=np.float32)
-        self.supercell_occ = np.asarray(arr["occ"], dtype=np.float32)
+        self.supercell_dw = np.array(arr["DW"], dtype=np.float32)    # copies: the records stay the caller's
+        self.supercell_occ = np.array(arr["occ"], dtype=np.float32)
         if self.debye_waller:  # per-element Gaussian displacement of x, y and z (msa.py:101-107)
             gen = rng if rng is not None else np.random
             for Z in np.unique(self.supercell_Z):
@@ -192,7 +192,8 @@ class MSAGPU:
                 dw = float(self.supercell_dw[idx][0])
                 self.supercell_xyz[idx] += (dw * gen.standard_normal(size=(len(idx), 3))).astype(np.float32)
 
-        self.dims = self.supercell_xyz.max(0) - self.supercell_xyz.min(0)
+        xyz = np.ascontiguousarray(self.supercell_xyz.T)   # a reduction along rows runs 20 times faster than down columns
+        self.dims = xyz.max(1) - xyz.min(1)
         self.max_angle = max_angle
         dims64 = self.dims[:2].astype(np.float64)
         if max_angle is None:
@@ -214,11 +215,12 @@ class MSAGPU:
         self._probes_dev = None
         self._probes_host = None
         self._slices_host = None
-        self.print_verbose(
-            "Simulation Parameters:\nSupercell dimensions xyz:%s (A)\nReal, Reciprocal space pixel "
-            "sizes:%s A, %s 1/A\nMax angle: %2.2f (rad)\nSampling: %s pixels,\nThermal Effects: %s"
-            % (np.round(self.dims, 3), np.round(self.pix_size, 3), np.round(self.kpix_size, 3),
-               self.max_ang, self.sampling, self.debye_waller))
+        if self.verbose:
+            self.print_verbose(
+                "Simulation Parameters:\nSupercell dimensions xyz:%s (A)\nReal, Reciprocal space pixel "
+                "sizes:%s A, %s 1/A\nMax angle: %2.2f (rad)\nSampling: %s pixels,\nThermal Effects: %s"
+                % (np.round(self.dims, 3), np.round(self.pix_size, 3), np.round(self.kpix_size, 3),
+                   self.max_ang, self.sampling, self.debye_waller))
 
     # ------------------------------------------------------------------ helpers
     @staticmethod
@@ -227,7 +229,7 @@ class MSAGPU:
             for field in ("x", "y", "z", "occ", "DW", "atomic_number"):
                 if field not in (supercell.dtype.names or ()):
                     raise ValueError("Supercell numpy array does not have required fields.")
-            return np.copy(supercell)
+            return supercell
         if isinstance(supercell, (str, os.PathLike)):
             if not os.path.exists(supercell):
                 raise FileNotFoundError("Path %s was not found." % supercell)
@@ -465,7 +467,9 @@ class MSAGPU:
         self.normalization = float(norm.item())
         self.psi_k = self.psi_k_device.cpu().numpy()
         self.apert = apert.cpu().numpy()
-        self.psi = (psi[0].cpu().numpy() / np.sqrt(self.normalization)).astype(np.complex64)
+        # in FP64 as numpy divides a complex by a real, the reciprocal rounded first
+        scaled = torch.view_as_real(psi[0]).double().mul_(float(1.0 / np.sqrt(self.normalization))).float()
+        self.psi = torch.view_as_complex(scaled).cpu().numpy()
 
     # ------------------------------------------------------------------ raster
     def generate_probe_positions(self, probe_step=np.array([0.1, 0.1]),
