@@ -443,14 +443,15 @@ __global__ void __launch_bounds__(256) integrate_slices_kernel(const double* pot
 }
 
 // Sites of one slice per workgroup, in input order: every workgroup reads all
-// depths (16 bytes a thread, from the L2 caches after the first), first to
+// depths (64 bytes a thread, from the L2 caches after the first), first to
 // count the sites before its slice, then to place its own, ranked by ballot
 // within a wavefront and by a running sum over wavefronts.  The reads grow with
 // S times A, but a workgroup's chain of steps only with A, and no list of a
 // site per step and slice has to be kept: 73,000 sites in 150 slices take
-// 73 us, 2.4 million in 310 3.6 ms, where the host's sorted lookup, stable
+// 30 us, 2.4 million in 310 1.4 ms, where the host's sorted lookup, stable
 // sort and three gathers took 7.3 and 350 ms.
 constexpr int kBinThreads = 1024;
+constexpr int kBinEach = 16;  // consecutive sites of a thread: 4 loads in flight a step (one took 73 us and 3.6 ms)
 
 // truncation as the host's conversion has it: INT_MIN for what an int cannot hold
 __device__ __forceinline__ int to_int(double v) {
@@ -464,26 +465,29 @@ bin_sites_kernel(const float* __restrict__ xyz, const float* __restrict__ z, con
   __shared__ int part[2][kBinThreads / 64];
   const int s = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const float first = bounds[0], lo = bounds[s], hi = bounds[s + 1];
-  const int steps = (A + 4 * kBinThreads - 1) / (4 * kBinThreads);
-  auto load = [&](int step, float (&v)[4]) {  // NaN past the end: in no slice
-    const int i = 4 * (step * kBinThreads + static_cast<int>(threadIdx.x));
-    if (i + 3 < A) {
-      const float4 f = *reinterpret_cast<const float4*>(z + i);
-      v[0] = f.x;
-      v[1] = f.y;
-      v[2] = f.z;
-      v[3] = f.w;
+  const int steps = (A + kBinEach * kBinThreads - 1) / (kBinEach * kBinThreads);
+  auto load = [&](int step, float (&v)[kBinEach]) {  // NaN past the end: in no slice
+    const int i = kBinEach * (step * kBinThreads + static_cast<int>(threadIdx.x));
+    if (i + kBinEach <= A) {
+#pragma unroll
+      for (int k = 0; k < kBinEach / 4; ++k) {
+        const float4 f = *reinterpret_cast<const float4*>(z + i + 4 * k);
+        v[4 * k] = f.x;
+        v[4 * k + 1] = f.y;
+        v[4 * k + 2] = f.z;
+        v[4 * k + 3] = f.w;
+      }
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = i + e < A ? z[i + e] : __builtin_nanf("");
+      for (int e = 0; e < kBinEach; ++e) v[e] = i + e < A ? z[i + e] : __builtin_nanf("");
     }
   };
   int before = 0;
   for (int step = 0; step < steps; ++step) {
-    float v[4];
+    float v[kBinEach];
     load(step, v);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) before += (v[e] >= first) & (v[e] < lo);
+    for (int e = 0; e < kBinEach; ++e) before += (v[e] >= first) & (v[e] < lo);
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
@@ -493,12 +497,12 @@ bin_sites_kernel(const float* __restrict__ xyz, const float* __restrict__ z, con
   for (int w = 0; w < kBinThreads / 64; ++w) base += part[0][w];
   if (threadIdx.x == 0) offsets[s] = base;
   for (int step = 0; step < steps; ++step) {
-    float v[4];
+    float v[kBinEach];
     load(step, v);
     int mine = 0, rank = 0, all = 0;
     const unsigned long long below = (1ull << lane) - 1;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < kBinEach; ++e) {
       const bool in = (v[e] >= lo) & (v[e] < hi);
       const unsigned long long m = __ballot(in);
       mine |= in << e;
@@ -513,9 +517,8 @@ bin_sites_kernel(const float* __restrict__ xyz, const float* __restrict__ z, con
       if (w == wave) rank += total;
       total += sums[w];
     }
-    for (int e = 0; e < 4; ++e) {
-      if (!(mine >> e & 1)) continue;
-      const long long i = 4ll * (static_cast<long long>(step) * kBinThreads + threadIdx.x) + e;
+    for (; mine; mine &= mine - 1) {
+      const long long i = static_cast<long long>(kBinEach) * (step * kBinThreads + threadIdx.x) + __ffs(mine) - 1;
       int a = 0, b = nZ;  // the first element not below this site's
       const long long own = Z[i];
       while (a < b) {

@@ -10,7 +10,7 @@ from namsa_amd import MSAGPU, structures
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("A,dz,wild", [(2, 2.0, False), (63, 0.5, True), (4095, 2.0, False), (4097, 1.0, True),
+@pytest.mark.parametrize("A,dz,wild", [(2, 2.0, False), (63, 0.5, True), (16383, 2.0, False), (16385, 1.0, True),
                                        (30011, 0.7, True)])
 def test_bins_match_host(gpu, A, dz, wild):
     print(f"bin sites A={A} dz={dz} wild={wild}", flush=True)
