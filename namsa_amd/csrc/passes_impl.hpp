@@ -618,8 +618,22 @@ struct SchedTable {
 // The base schedule (entry 0 of a table) serves every op; the alternatives
 // only replace the hot ops (row STEP, column PROP and READOUT) and defer the
 // rest to the base schedule.
-template <class S, class Base>
+//
+// Many: the same transform without the prefetch, which STEP launches of more
+// than a workgroup per CU take.  The prefetch brings a workgroup's first rows
+// in sooner and costs registers (slice step at 128^2, with it and without: 1
+// image 7.49 and 7.62 us, 32 images 8.62 and 8.67, 48 images 9.89 and 9.69, 300
+// images 25.0 and 24.4, 1089 images 69.7 and 68.6).  The bits are the same.
+template <class S, class Base, class Many = void>
 int launch_row(int op, const RowArgs& a, hipStream_t st) {
+  if constexpr (!std::is_void<Many>::value) {
+    static_assert(S::PF && !Many::PF && Many::N == S::N && Many::E == S::E && Many::CT == S::CT &&
+                      std::is_same<typename Many::RL, typename S::RL>::value,
+                  "a form for many rows only drops the prefetch");
+    constexpr int G = kRowThreads / (S::N / S::E);
+    if (op == ROW_STEP && a.n_rows > static_cast<long long>(G) * device_cu_count())
+      return launch_row_op<Many, ROW_STEP>(a, st);
+  }
   if (op == ROW_STEP) return launch_row_op<S, ROW_STEP>(a, st);
   if constexpr (std::is_same<S, Base>::value) {
     if (op == ROW_INV) return launch_row_op<S, ROW_INV>(a, st);

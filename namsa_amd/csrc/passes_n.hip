@@ -22,7 +22,7 @@ using C2 = ColS<128, 8, Radices<8, 4, 4>, 16, false, false, false, false, 4, tru
 using R2 = RowS<128, 8, Radices<8, 4, 4>, false, false, false, 6>;
 using C2N = ColS<128, 8, Radices<8, 4, 4>, 8, false, false, false, false, 5, true, true>;
 static const RowSchedEntry kRows[] = {{"e8.r844", launch_row<R0, R0>},
-                                      {"e8.r844.pf", launch_row<R1, R0>},
+                                      {"e8.r844.pf", launch_row<R1, R0, R0>},
                                       {"e8.r844.w6", launch_row<R2, R0>}};
 static const ColSchedEntry kCols[] = {{"e8.r844.c16", launch_col<C0, C0>, 16},
                                       {"e8.r844.c8.pf", launch_col<C1, C0>, 8},
