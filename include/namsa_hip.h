@@ -460,6 +460,11 @@ int namsa_fno_head_backward(const float* x, const float* Q1, const float* bq1, c
 int namsa_spectral_pack(const void* psi_c, const void* psi_0, const void* vhat, const int* vidx, int nv, int B, int Ny,
                         int Nx, int r0, int c0, int H, int W, const float* kmax, float s, float phase_scale,
                         const float* thick, float thick_scale, float vscale, int opts, float* u, void* stream);
+/* Rows idx[0 .. rows) (device memory, each inside its tensors) of up to 8
+ * tensors, copied to consecutive rows: src[i], dst[i] device pointers with rows
+ * of row_bytes[i] bytes (4-byte words); the three arrays are host memory. */
+int namsa_gather_rows(const void* const* src, void* const* dst, const long long* row_bytes, int tensors,
+                      const long long* idx, int rows, void* stream);
 int namsa_spectral_loss(const float* out, const void* psi_c, const float* target, int B, int Ny, int Nx, int r0,
                         int c0, int H, int W, float s, double* sums, float* gout, void* stream);
 int namsa_spectral_apply(const float* out, const void* psi_c, int B, int Ny, int Nx, int r0, int c0, int H, int W,

@@ -78,6 +78,7 @@ SIGNATURES = {
     "namsa_potential_record": (_i, [_vp, _i, _i, _i, _d, _d, _vp, _vp, _vp]),
     "namsa_spectral_pack": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _f, _f, _vp, _f, _f, _i,
                                  _vp, _vp]),
+    "namsa_gather_rows": (_i, [_vp, _vp, _vp, _i, _vp, _i, _vp]),
     "namsa_spectral_loss": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _vp, _vp, _vp]),
     "namsa_spectral_apply": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _vp, _vp]),
     "namsa_real_to_complex": (_i, [_vp, _i, _i, _i, _f, _i, _vp, _vp]),

@@ -28,6 +28,7 @@ so the mixing is one batched [2C x 2C] x [2C x B] GEMM over the m*m modes).
 """
 from __future__ import annotations
 
+import ctypes
 import math
 
 import numpy as np
@@ -289,10 +290,11 @@ class FnoNet:
         self._gemm(_addr(self.Zp), (0, m2, 1), _addr(self.Fx), (0, 1, m2), dest, (0, W, 1),
                    CB * H, W, m2, alpha=alpha, beta=beta, gelu=gelu, P=P)
 
-    def _rows(self, x, cin, Wt, transposed, B, out, Zp=None, bias=None, alpha=1.0, pre_in=None, pre_out=None, zalpha=1.0,
-              Z=None):
-        call("namsa_fno_rows", x, cin, Zp, ptr(self.fx_bf), ptr(self.fxT_bf), Wt, transposed, bias, np.float32(alpha), pre_in,
-             pre_out, np.float32(zalpha), B, self.H, self.W, self.Wp, out, Z, self.st)
+    def _rows(self, x, cin, Wt, transposed, B, out, Zp=None, bias=None, alpha=1.0, pre_in=None, pre_out=None,
+              zalpha=1.0, Z=None):
+        """A layer's row-local work on x [cin][B*H*W] (namsa_fno_rows)."""
+        call("namsa_fno_rows", x, cin, Zp, ptr(self.fx_bf), ptr(self.fxT_bf), Wt, transposed, bias,
+             np.float32(alpha), pre_in, pre_out, np.float32(zalpha), B, self.H, self.W, self.Wp, out, Z, self.st)
 
     # ------------------------------------------------------------------ passes
     def forward(self, B):
@@ -371,10 +373,10 @@ class FnoNet:
 
     def forward_graph(self, B):
         """forward_fused(B) replayed from a HIP graph captured on first use for
-        this B (about 26 launches per pass: issued one by one from the host
-        they cost more time than the kernels take at 256^2).  The graph reads
-        u and writes out in place; the weights are read at replay time, so
-        loading new parameters needs no recapture."""
+        this B (17 launches per pass: issued one by one from the host they
+        cost more time than the kernels of a few samples take at 256^2).  The
+        graph reads u and writes out in place; the weights are read at replay
+        time, so loading new parameters needs no recapture."""
         torch = _torch()
         g = self._graphs.get(B)
         if g is None:
@@ -412,8 +414,8 @@ class FnoNet:
         go, ones = ptr(self.gout), ptr(self.ones)
         ga, gb = self.ga, self.gb
         if self.head_ok(B):
-            call("namsa_fno_head_backward", ptr(self.xs[L]), self._p("Q1"), self._p("bq1"), self._p("Q2"), go, n, ptr(ga),
-                 self._g("Q1"), self._g("bq1"), self._g("Q2"), self._g("bq2"), self.st)
+            call("namsa_fno_head_backward", ptr(self.xs[L]), self._p("Q1"), self._p("bq1"), self._p("Q2"), go, n,
+                 ptr(ga), self._g("Q1"), self._g("bq1"), self._g("Q2"), self._g("bq2"), self.st)
         else:
             self._gemm(go, (0, n, 1), ptr(self.h), (0, 1, n), self._g("Q2"), (0, Hq, 1), 2, Hq, n, split=sp)
             self._gemm(go, (0, n, 1), ones, (0, 1, 0), self._g("bq2"), (0, 1, 1), 2, 1, n, split=sp)
@@ -692,6 +694,26 @@ class SpectralCorrector:
         return self.apply(psi_c, B, cbed)
 
 
+def _gather(tensors, idx):
+    """Rows idx of each tensor, as index_select gives them, in one launch."""
+    torch = _torch()
+    host = np.asarray(idx)
+    dev = tensors[0].device
+    ii = torch.as_tensor(host, device=dev)
+    if not (ii.dtype == torch.int64 and ii.dim() == 1 and 0 < len(ii) <= 65535 and dev.type == "cuda"
+            and all(t.device == dev and t.is_contiguous() and t.element_size() % 4 == 0 and t.numel() and t.dim()
+                    and not t.requires_grad for t in tensors)
+            and host.min() >= 0 and host.max() < min(len(t) for t in tensors)):
+        return tuple(t.index_select(0, ii) for t in tensors)
+    out = tuple(torch.empty((len(ii), *t.shape[1:]), dtype=t.dtype, device=dev) for t in tensors)
+    n = len(tensors)
+    call("namsa_gather_rows", (ctypes.c_void_p * n)(*(t.data_ptr() for t in tensors)),
+         (ctypes.c_void_p * n)(*(t.data_ptr() for t in out)),
+         (ctypes.c_longlong * n)(*(t.numel() // len(t) * t.element_size() for t in tensors)), n, ptr(ii), len(ii),
+         stream_handle())
+    return out
+
+
 class SpectralPairPool:
     """Training pairs resident in HBM: per coarsening factor the coarse exit
     spectra, and shared by every factor the vacuum spectra, the fine CBEDs
@@ -748,10 +770,7 @@ class SpectralPairPool:
         return len(self.th)
 
     def batch(self, idx, factor):
-        torch = _torch()
-        ii = torch.as_tensor(np.asarray(idx), device=self.P0.device)
-        return (self.PC[factor].index_select(0, ii), self.P0.index_select(0, ii), self.F.index_select(0, ii),
-                self.TH.index_select(0, ii), self.VI.index_select(0, ii), self.KM.index_select(0, ii))
+        return _gather((self.PC[factor], self.P0, self.F, self.TH, self.VI, self.KM), idx)
 
 
 def spectral_batch_loss(corr, pool, idx, grad=False):

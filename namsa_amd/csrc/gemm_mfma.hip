@@ -10,15 +10,15 @@
 // 32-channel or 32-mode dimension), so N <= 32 takes 128 x 32 tiles, M <= 32
 // takes 32 x 128 tiles and the rest 64 x 64 -- no wavefront idles on a
 // 32-wide side -- and batches of many items that each fit one 32 x 32 block
-// take one wavefront per item.  Operand tiles of K = 32 are staged through LDS as bf16 with
-// k contiguous: the unit-stride axis is read with 16-byte loads (at any 4-byte
-// aligned address), and the next K tile is loaded into
-// registers while the matrix cores work on the current one.  MFMA operands
-// come out of LDS as 16-byte reads.  Pointwise layers over many columns run without
-// LDS (gemm_pointwise_kernel).  With split_k > 1 the K range is divided
-// over workgroups and partial products are added to C with FP32 atomics (C
-// must then already hold beta*C); gemm_split_kernel takes the small products
-// over a long contiguous K.
+// take one workgroup per item.  Operand tiles of K = 32 are staged through LDS
+// as bf16 with k contiguous: the unit-stride axis is read with 16-byte loads
+// (at any 4-byte aligned address), and the next K tile is loaded into registers
+// while the matrix cores work on the current one.  MFMA operands come out of
+// LDS as 16-byte reads.  Pointwise layers over many columns run without LDS
+// (gemm_pointwise_kernel).  With split_k > 1 the K range is divided over
+// workgroups and partial products are added to C with FP32 atomics (C must then
+// already hold beta*C); gemm_split_kernel takes the small products over a long
+// contiguous K.
 //
 // MFMA 32x32x16 operand layout (lane l, 8 bf16 per operand register set):
 //   A: row l%32, k = 8*(l/32) + e      B: column l%32, k = 8*(l/32) + e
@@ -224,7 +224,7 @@ __device__ __forceinline__ void store_block(const GemmArgs& g, long long b, cons
 }
 
 // Batched products whose every matrix fits one MFMA block (M <= 32, N <= 32;
-// the corrector's mode-space y transforms, thousands of 32 x 32 x H items):
+// the y transforms of a corrector of other than 16 modes, hundreds of items):
 // one workgroup per batch item, its four wavefronts taking every fourth
 // K step of 16 with the operands read straight into the MFMA layout, the
 // partial accumulators summed through LDS.  Splitting K shortens each

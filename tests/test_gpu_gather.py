@@ -1,0 +1,24 @@
+"""A minibatch gathered in one launch against index_select, bit for bit: rows
+of whole and of odd numbers of 16-byte words, scalars, repeated and reversed
+rows, more than a workgroup's share a row; tensors it does not take fall back."""
+import numpy as np
+import pytest
+
+from namsa_amd import corrector as K
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape,idx", [((1,), [0]), ((7,), [3, 3, 0]), ((65, 67), [5, 4, 0, 5]),
+                                       ((256, 256), list(range(5, -1, -1)))])
+def test_gather_equals_index_select(gpu, shape, idx):
+    import torch
+    print(f"gather {shape} {idx}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(len(idx))
+    real = torch.randn((6, *shape), device=gpu, generator=g)
+    tensors = (torch.complex(real, -real), real, torch.arange(6, device=gpu, dtype=torch.int32), real[:, 0].contiguous(),
+               torch.randn((7, 3), device=gpu, generator=g)[1:], real.double())
+    for t in (tensors, (real.half(), real), (real.transpose(0, -1).contiguous().transpose(0, -1), real)):
+        for a, b in zip(K._gather(t, idx), t):
+            want = b.index_select(0, torch.as_tensor(idx, device=gpu))
+            assert a.dtype == want.dtype and a.shape == want.shape and torch.equal(a, want)
