@@ -650,13 +650,35 @@ int launch_row(int op, const RowArgs& a, hipStream_t st) {
 // -> 9.6, 1024^2 20.1 -> 17.5; at two tasks per CU the two are equal or the
 // wide one is ahead).  Same operations per column: the bits do not depend on
 // it, as long as both read the propagator the same way (PG).
-template <class S, class Base, class Narrow = void>
+//
+// Even: the same transform in a persistent form (a workgroup keeps its strip
+// and runs through images), which PROP launches take that give its resident
+// workgroups an image each at most (a twentieth more passes unnoticed), or up to
+// three to within a tenth: it has no last wave to wait for, while a few waves of
+// single tasks end in a part one (slice step, tasks and persistent: 256^2, 24
+// images 13.7 and 13.4 us, 110 images 37.2 and 36.0, 170 images 53.0 and 50.5,
+// but 125 images 41.9 and 43.6; 192^2, 92 images 22.3 and 21.6, 100 images 24.4
+// and 23.1, but 110 images 25.6 and 28.6).
+template <class S, class Base, class Narrow = void, class Even = void>
 int launch_col(int op, ColArgs& a, hipStream_t st) {
   if constexpr (!std::is_void<Narrow>::value) {
     static_assert(Narrow::C < S::C && Narrow::PG == S::PG && std::is_same<typename Narrow::F, typename S::F>::value,
                   "a narrow form only changes the strip");
     const long long strips = (a.band_hi + Narrow::C - 1) / Narrow::C - a.band_lo / Narrow::C;
     if (op == COL_PROP && strips * a.B <= device_cu_count()) return launch_col_op<Narrow, COL_PROP>(a, st);
+  }
+  if constexpr (!std::is_void<Even>::value) {
+    static_assert(Even::W == 0 && Even::PG == S::PG && std::is_same<typename Even::F, typename S::F>::value,
+                  "a persistent form only changes who takes which task");
+    if (op == COL_PROP) {
+      static const int cap = persistent_cap(col_kernel<Even, COL_PROP>, Even::threads());
+      const int strips = (a.band_hi + Even::C - 1) / Even::C - a.band_lo / Even::C;
+      const long long sets = strips > 0 ? cap / strips : 0;
+      const long long rounds = sets > 0 ? a.B / sets : 4, left = sets > 0 ? a.B % sets : 0;
+      const bool even = rounds == 0 || (rounds <= 3 && 20 * left <= sets) ||
+                        (rounds <= 2 && 10LL * a.B >= 9 * (rounds + 1) * sets);
+      if (even) return launch_col_op<Even, COL_PROP>(a, st);
+    }
   }
   if (op == COL_PROP) return launch_col_op<S, COL_PROP>(a, st);
   // the multi-workgroup schedules' readout (one task per (strip, image),

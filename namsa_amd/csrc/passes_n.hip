@@ -46,7 +46,7 @@ static const ColSchedEntry kCols[] = {{"e12.r3444.c16", launch_col<C0, C0>, 16},
                                       {"e12.r3444.c8.pf", launch_col<C1, C0>, 8},
                                       {"e12.r12.4.4.c16", launch_col<C2, C0>, 16},
                                       {"e12.r12.4.4.c8.pf", launch_col<C3, C0>, 8},
-                                      {"e12.r12.4.4.c16.sb.w4.i2", launch_col<C4, C0, C4N>, 16}};
+                                      {"e12.r12.4.4.c16.sb.w4.i2", launch_col<C4, C0, C4N, C2>, 16}};
 #elif NAMSA_PASS_N == 256
 using R0 = RowS<256, 8, Radices<8, 8, 4>, false, false>;
 using R1 = RowS<256, 8, Radices<8, 8, 4>, true, false>;
@@ -64,7 +64,7 @@ static const RowSchedEntry kRows[] = {{"e8.r884", launch_row<R0, R0>},
 static const ColSchedEntry kCols[] = {{"e8.r884.c16", launch_col<C0, C0>, 16},
                                       {"e8.r884.c8.pf", launch_col<C1, C0>, 8},
                                       {"e16.r16.16.c16.pf", launch_col<C2, C0>, 16},
-                                      {"e8.r884.c8.sb.w6.i2", launch_col<C3, C0, C3N>, 8}};
+                                      {"e8.r884.c8.sb.w6.i2", launch_col<C3, C0, C3N, C1>, 8}};
 #elif NAMSA_PASS_N == 384
 using R0 = RowS<384, 12, Radices<3, 2, 4, 4, 4>, false, false>;
 using R1 = RowS<384, 12, Radices<3, 2, 4, 4, 4>, true, false>;

@@ -11,8 +11,9 @@ from namsa_amd import autotune
 
 pytestmark = pytest.mark.gpu
 
-# batches on both sides of one narrow-strip task per CU, and of one image per workgroup
-BATCH = {128: 70, 192: 50, 256: 40, 384: 24, 512: 14, 768: 7, 1024: 9, 2048: 4}
+# batches on both sides of one narrow-strip task per CU, and of one image per
+# workgroup; at 192 and 256 the whole batch fills a persistent launch evenly
+BATCH = {128: 70, 192: 92, 256: 56, 384: 24, 512: 14, 768: 7, 1024: 9, 2048: 4}
 
 
 @pytest.mark.parametrize("mode", [L.OUT_CBED, L.OUT_EXIT])
