@@ -30,6 +30,7 @@
 
 #include "common.hpp"
 #include "gelu.hpp"
+#include "gemm_paths.hpp"
 #include "namsa_hip.h"
 
 namespace namsa {
@@ -384,7 +385,7 @@ __global__ void __launch_bounds__(256) gemm_split_kernel(GemmArgs g, int k_per, 
 // first product.  Reads and writes are buffer accesses: a scalar row offset
 // and one lane offset (with pointers the 64-bit addresses took 250 registers),
 // rows past K read 0 and rows past M are not written, being past the buffer's
-// end (the launcher checks sBk, sCi >= N and 31-bit sizes).  The products run
+// end (pointwise_fits: no offset wraps).  The products run
 // over k in the order of the staged kernel.  Over 462,400 columns: 32
 // x 32 with bias 47 -> 32 us, with beta 57 -> 31, 32 x 7 44 -> 16, 64 x 32 with
 // GELU 109 -> 82 (296 MB).
@@ -471,6 +472,7 @@ int launch_pointwise(const GemmArgs& g, hipStream_t st) {
   // blocks per wavefront: 4 with a bias (its 16 reads per 32 rows are then
   // paid once per 128 columns) and for K = 32, else 2
   constexpr int PB = KS == 2 ? 4 : 2;
+  static_assert(128 * 4 <= kPointwiseCols, "pointwise_fits counts the columns of a workgroup");
   const auto grid = [&](int pb) { return dim3((g.N + 128 * pb - 1) / (128 * pb)); };
   if (g.bias_mode == 1)
     hipLaunchKernelGGL((gemm_pointwise_kernel<MT, KS, 4, true>), grid(4), dim3(256), 0, st, g);
@@ -530,12 +532,13 @@ int namsa_gemm_bf16(const float* A, long long sAb, long long sAi, long long sAk,
     if (M <= 32) return N <= 32 ? launch_split<1, 1>(g, st) : launch_split<1, 2>(g, st);
     return N <= 32 ? launch_split<2, 1>(g, st) : launch_split<2, 2>(g, st);
   }
-  const long long buf_max = 0x7fffffffLL / 4;
-  if (batch == 1 && split_k == 1 && sBj == 1 && sCj == 1 && M <= 64 && K <= 64 && N >= 8192 && sBk >= N && sCi >= N &&
-      K * sBk <= buf_max && M * sCi <= buf_max) {
-    if (K <= 16) return M <= 32 ? launch_pointwise<1, 1>(g, st) : launch_pointwise<2, 1>(g, st);
-    if (K <= 32) return M <= 32 ? launch_pointwise<1, 2>(g, st) : launch_pointwise<2, 2>(g, st);
-    return M <= 32 ? launch_pointwise<1, 4>(g, st) : launch_pointwise<2, 4>(g, st);
+  if (batch == 1 && split_k == 1 && sBj == 1 && sCj == 1 && N >= 8192 && pointwise_fits(M, N, K, sBk, sCi)) {
+    const bool one = pointwise_mt(M) == 1;
+    switch (pointwise_ks(K)) {
+      case 1: return one ? launch_pointwise<1, 1>(g, st) : launch_pointwise<2, 1>(g, st);
+      case 2: return one ? launch_pointwise<1, 2>(g, st) : launch_pointwise<2, 2>(g, st);
+      default: return one ? launch_pointwise<1, 4>(g, st) : launch_pointwise<2, 4>(g, st);
+    }
   }
   if (N <= 32) return launch_gemm<4, 1>(g, st);
   if (M <= 32) return launch_gemm<1, 4>(g, st);

@@ -46,3 +46,20 @@ def test_pointwise_products(gpu, M, N, K, pad, off, beta, bias, gelu):
     else:
         assert (np.abs(got[:, :N] - pre) <= bound).all()
     assert np.array_equal(got[:, N:], rows(C0, M)[:, N:]) and np.array_equal(Cd[:off].cpu().numpy(), C0[:off])
+
+
+@pytest.mark.parametrize("M,N", [(1, 2 ** 28), (2, 2 ** 27)])
+def test_products_wider_than_the_pointwise_offsets(gpu, M, N):
+    """Rows so long that a 32-bit offset of row 31 would wrap into row 0: K = 1,
+    so each value is one product of two bf16 numbers, exact in float32."""
+    import torch
+
+    print(f"wide gemm M={M} N={N}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(M)
+    A = torch.randn((M, 1), device=gpu, generator=g).to(torch.bfloat16).float()
+    B = torch.randn(N, device=gpu, generator=g).to(torch.bfloat16).float()
+    C = torch.full((M, N), np.nan, device=gpu)
+    L.call("namsa_gemm_bf16", L.ptr(A), 0, 1, 1, L.ptr(B), 0, N, 1, L.ptr(C), 0, N, 1, M, N, 1, 1, 1, np.float32(1.0),
+           np.float32(0.0), None, 0, 0, None, L.stream_handle())
+    for i in range(M):
+        assert torch.equal(C[i], A[i] * B), i
