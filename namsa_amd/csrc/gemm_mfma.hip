@@ -302,15 +302,15 @@ __global__ void __launch_bounds__(256) gemm_split_kernel(GemmArgs g, int k_per, 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long long b = blockIdx.y;
   const int row = lane & 31, kh = 8 * (lane >> 5);
-  const int k_begin = blockIdx.x * k_per, k_end = min(g.K, k_begin + k_per);
+  const int k_begin = blockIdx.x * k_per, k_len = split_len(g.K, k_begin, k_per);
   // lanes past the last row or column read that row: what they add to goes
   // into values that are not stored
   const float* A[MT];
   const float* B[NT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) A[i] = g.A + b * g.sAb + min(32 * i + row, g.M - 1) * g.sAi + kh;
+  for (int i = 0; i < MT; ++i) A[i] = g.A + b * g.sAb + min(32 * i + row, g.M - 1) * g.sAi + k_begin + kh;
 #pragma unroll
-  for (int j = 0; j < NT; ++j) B[j] = g.B + b * g.sBb + min(32 * j + row, g.N - 1) * g.sBj + kh;
+  for (int j = 0; j < NT; ++j) B[j] = g.B + b * g.sBb + min(32 * j + row, g.N - 1) * g.sBj + k_begin + kh;
   f32x16 acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -327,11 +327,11 @@ __global__ void __launch_bounds__(256) gemm_split_kernel(GemmArgs g, int k_per, 
 #pragma unroll
     for (int r = 0; r < 16; ++r) total[i][r] = 0.0f;
 #pragma unroll 2
-  for (int k0 = k_begin + 32 * wave; k0 < k_end; k0 += 128) {
+  for (int k0 = 32 * wave; k0 < k_len; k0 += 128) {
     bf16x8 a[MT][2], c[NT][2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int left = k_end - k0 - kh - 16 * h;
+      const int left = k_len - k0 - kh - 16 * h;
 #pragma unroll
       for (int i = 0; i < MT; ++i) a[i][h] = load_k8(A[i] + k0 + 16 * h, left);
 #pragma unroll
@@ -483,12 +483,9 @@ int launch_pointwise(const GemmArgs& g, hipStream_t st) {
 
 template <int MT, int NT, bool SUMS = false>
 int launch_split(const GemmArgs& g, hipStream_t st, float* sums = nullptr) {
-  // one workgroup per CU, each at least one step of 32 k per wavefront
-  const int cus = device_cu_count();
-  const int groups = std::max(1, std::min((g.K + 127) / 128, (cus + g.batch - 1) / g.batch));
-  const int k_per = ((g.K + groups - 1) / groups + 127) / 128 * 128;
-  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, SUMS>), dim3((g.K + k_per - 1) / k_per, g.batch), dim3(256), 0, st, g,
-                     k_per, sums);
+  const SplitPlan plan = split_plan(g.K, g.batch, device_cu_count());
+  hipLaunchKernelGGL((gemm_split_kernel<MT, NT, SUMS>), dim3(plan.groups, g.batch), dim3(256), 0, st, g, plan.k_per,
+                     sums);
   return check_hip(hipGetLastError(), "gemm_split_kernel launch");
 }
 
@@ -528,7 +525,7 @@ int namsa_gemm_bf16(const float* A, long long sAb, long long sAi, long long sAk,
     hipLaunchKernelGGL(gemm_small_kernel, dim3(static_cast<unsigned>(batch)), dim3(256), 0, st, g);
     return check_hip(hipGetLastError(), "gemm_small_kernel launch");
   }
-  if (split_k > 1 && sAk == 1 && sBk == 1 && M <= 64 && N <= 64) {
+  if (split_k > 1 && sAk == 1 && sBk == 1 && M <= 64 && N <= 64 && K <= kSplitMaxK) {
     if (M <= 32) return N <= 32 ? launch_split<1, 1>(g, st) : launch_split<1, 2>(g, st);
     return N <= 32 ? launch_split<2, 1>(g, st) : launch_split<2, 2>(g, st);
   }
@@ -546,7 +543,7 @@ int namsa_gemm_bf16(const float* A, long long sAb, long long sAi, long long sAk,
 }
 
 int namsa_weight_grad(const float* gy, const float* x, long long n, int M, int N, float* gW, float* gb, void* stream) {
-  if (!gy || !x || !gW || !gb || n <= 0 || n > 0x7fffff00LL || M < 1 || M > 32 || N < 1 || N > 32)
+  if (!gy || !x || !gW || !gb || n <= 0 || n > kSplitMaxK || M < 1 || M > 32 || N < 1 || N > 32)
     return fail(kErrArg, "namsa_weight_grad: null argument, n=%lld or M=%d N=%d outside 1..32", n, M, N);
   const GemmArgs g{gy, 0, n, 1, x, 0, 1, n, gW, 0, N, 1, M, N, static_cast<int>(n), 1, 2, 1.0f, 0.0f, nullptr, 0, 0,
                    nullptr};

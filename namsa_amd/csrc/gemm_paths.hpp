@@ -22,4 +22,23 @@ constexpr bool pointwise_fits(int M, int N, int K, long long sBk, long long sCi)
          sBk <= (INT_MAX - 4 * kPointwiseCols) / (64 * pointwise_ks(K)) && sCi <= INT_MAX / (128 * pointwise_mt(M));
 }
 
+// gemm_split_kernel's share of K: workgroup x takes split_len(K, x * k_per,
+// k_per) values from x * k_per on, in steps of 128 that stay below 2^31 from
+// kSplitMaxK down.  One workgroup per CU, each at least one step of 32 k per
+// wavefront.
+constexpr int kSplitMaxK = INT_MAX - 255;
+
+struct SplitPlan {
+  int groups, k_per;
+};
+
+constexpr SplitPlan split_plan(int K, int batch, int cus) {
+  const long long most = (cus + batch - 1LL) / batch, steps = (K + 127LL) / 128;
+  const long long want = steps < most ? steps : most;
+  const long long k_per = ((K + want - 1) / want + 127) / 128 * 128;
+  return {static_cast<int>((K + k_per - 1) / k_per), static_cast<int>(k_per)};
+}
+
+constexpr int split_len(int K, int k_begin, int k_per) { return K - k_begin < k_per ? K - k_begin : k_per; }
+
 }  // namespace namsa

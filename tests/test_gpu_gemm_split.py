@@ -58,3 +58,17 @@ def test_weight_grad(gpu, M, N, n):
     a, w = bf16(gy), np.concatenate([bf16(x), np.ones((1, n))])
     err = np.linalg.norm(got - C0 - a @ w.T) / np.linalg.norm(np.abs(a) @ np.abs(w).T)
     assert err < 2e-5, err
+
+
+def test_weight_grad_over_the_largest_k(gpu):
+    """The last workgroup's share ends at 2^31 - 256: only the last 1000 values
+    of one vector, taken as both operands, are not 0, so the sums are exact."""
+    import torch
+
+    n = 2 ** 31 - 256
+    print(f"weight grad n={n}", flush=True)
+    v = torch.zeros(n, device=gpu)
+    v[-1000:] = 2.0
+    out = torch.zeros(2, device=gpu)
+    L.call("namsa_weight_grad", L.ptr(v), L.ptr(v), n, 1, 1, L.ptr(out), L.ptr(out[1:]), L.stream_handle())
+    assert out.tolist() == [4000.0, 2000.0]
