@@ -695,14 +695,15 @@ class SpectralCorrector:
 
 
 def _gather(tensors, idx):
-    """Rows idx of each tensor, as index_select gives them, in one launch."""
+    """Rows idx of each tensor, as index_select gives them, in one launch where
+    the bytes in memory are the values (no lazily conjugated or negated view)."""
     torch = _torch()
     host = np.asarray(idx)
     dev = tensors[0].device
     ii = torch.as_tensor(host, device=dev)
     if not (ii.dtype == torch.int64 and ii.dim() == 1 and 0 < len(ii) <= 65535 and dev.type == "cuda"
             and all(t.device == dev and t.is_contiguous() and t.element_size() % 4 == 0 and t.numel() and t.dim()
-                    and not t.requires_grad for t in tensors)
+                    and not (t.requires_grad or t.is_conj() or t.is_neg()) for t in tensors)
             and host.min() >= 0 and host.max() < min(len(t) for t in tensors)):
         return tuple(t.index_select(0, ii) for t in tensors)
     out = tuple(torch.empty((len(ii), *t.shape[1:]), dtype=t.dtype, device=dev) for t in tensors)

@@ -22,3 +22,16 @@ def test_gather_equals_index_select(gpu, shape, idx):
         for a, b in zip(K._gather(t, idx), t):
             want = b.index_select(0, torch.as_tensor(idx, device=gpu))
             assert a.dtype == want.dtype and a.shape == want.shape and torch.equal(a, want)
+
+
+@pytest.mark.parametrize("lazy", ["conj", "neg"])
+def test_gather_resolves_lazy_views(gpu, lazy):
+    """Views that torch marks as conjugated or negated instead of computing
+    them are contiguous; their rows have the values, as index_select gives them."""
+    import torch
+    z = torch.randn((5, 6, 4), dtype=torch.complex64, device=gpu, generator=torch.Generator(device=gpu).manual_seed(1))
+    view = z.conj() if lazy == "conj" else torch._neg_view(z.real.contiguous())
+    assert view.is_contiguous() and (view.is_conj() or view.is_neg())
+    got, = K._gather((view,), [4, 0, 2])
+    want = view.index_select(0, torch.tensor([4, 0, 2], device=gpu))
+    assert torch.equal(got, want) and float(want.abs().max()) > 0
