@@ -702,6 +702,7 @@ def _gather(tensors, idx):
     dev = tensors[0].device
     ii = torch.as_tensor(host, device=dev)
     if not (ii.dtype == torch.int64 and ii.dim() == 1 and 0 < len(ii) <= 65535 and dev.type == "cuda"
+            and dev.index == torch.cuda.current_device()    # the launch goes to its current stream
             and all(t.device == dev and t.is_contiguous() and t.element_size() % 4 == 0 and t.numel() and t.dim()
                     and not (t.requires_grad or t.is_conj() or t.is_neg()) for t in tensors)
             and host.min() >= 0 and host.max() < min(len(t) for t in tensors)):

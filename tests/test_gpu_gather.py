@@ -35,3 +35,14 @@ def test_gather_resolves_lazy_views(gpu, lazy):
     got, = K._gather((view,), [4, 0, 2])
     want = view.index_select(0, torch.tensor([4, 0, 2], device=gpu))
     assert torch.equal(got, want) and float(want.abs().max()) > 0
+
+
+def test_gather_leaves_other_devices_to_torch(gpu, monkeypatch):
+    """The launch goes to the current device's stream: tensors of another
+    device are left to index_select, which runs on theirs."""
+    import torch
+    t = torch.arange(12.0, device=gpu).reshape(4, 3)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: gpu.index + 1)
+    monkeypatch.setattr(K, "call", lambda name, *a: pytest.fail(name))
+    got, = K._gather((t,), [3, 1])
+    assert got.tolist() == [[9.0, 10.0, 11.0], [3.0, 4.0, 5.0]]
