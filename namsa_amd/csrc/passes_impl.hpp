@@ -682,9 +682,17 @@ int launch_col(int op, ColArgs& a, hipStream_t st) {
   }
   if (op == COL_PROP) return launch_col_op<S, COL_PROP>(a, st);
   // the multi-workgroup schedules' readout (one task per (strip, image),
-  // detector reductions per task) is 20-50% slower than the base schedule's
+  // detector reductions per task) is 20-50% slower than a persistent one's, so
+  // it goes to the persistent form where the base schedule's transform is
+  // another (192^2, 910 images, two slices and two detectors: 421 us, base 440),
+  // else to the base schedule (256^2, 448 images: base 348, persistent 378)
   if (op == COL_READOUT) {
-    if constexpr (S::W > 0)
+    if constexpr (!std::is_void<Even>::value) {
+      if constexpr (!std::is_same<typename Even::F, typename Base::F>::value)
+        return launch_col_op<Even, COL_READOUT>(a, st);
+      else
+        return launch_col<Base, Base>(op, a, st);
+    } else if constexpr (S::W > 0)
       return launch_col<Base, Base>(op, a, st);
     else
       return launch_col_op<S, COL_READOUT>(a, st);
