@@ -86,3 +86,10 @@ def test_head_equals_separate_products(gpu, n):
         want, size = a @ b.T, a.abs() @ b.abs().T
         err = (grads[k].reshape(want.shape) - want).abs()
         assert (err <= n * 2.0 ** -23 * size).all(), (k, float((err / size).max()))
+
+
+@pytest.mark.parametrize("H,W,cin,B", [(16, 385, 7, 1), (17, 800, 7, 1), (16, 768, 3, 2)])
+def test_rows_wider_than_a_workgroup(gpu, H, W, cin, B):
+    """More tiles a row than a workgroup's wavefronts hold: several runs a row
+    (two, three uneven ones, two full ones), the row DFT carried from run to run."""
+    test_row_kernels_equal_separate_products(gpu, H, W, cin, B)
