@@ -207,8 +207,9 @@ class FnoNet:
         self.B_fused = B
 
     def rows_ok(self, B):
-        """The row kernels of training are compiled for 32 channels and 16 modes and index 32 channels in 31 bits."""
-        return (self.C, self.m) == (32, 16) and self.cin <= 16 and 128 * B * self.H * self.W < 2 ** 31
+        """The row kernels of training are compiled for 32 channels and 16 modes and index 32 channels
+        of the activations and of the row DFTs (32 values a row) in 31 bits."""
+        return (self.C, self.m) == (32, 16) and self.cin <= 16 and 128 * B * self.H * max(self.W, 32) < 2 ** 31
 
     def head_ok(self, B):
         """The head's kernels of training are compiled for 32 and 64 channels and index 32 channels in 31 bits."""
