@@ -229,7 +229,7 @@ class MSAGPU:
             for field in ("x", "y", "z", "occ", "DW", "atomic_number"):
                 if field not in (supercell.dtype.names or ()):
                     raise ValueError("Supercell numpy array does not have required fields.")
-            return supercell
+            return np.asarray(supercell)
         if isinstance(supercell, (str, os.PathLike)):
             if not os.path.exists(supercell):
                 raise FileNotFoundError("Path %s was not found." % supercell)

@@ -222,3 +222,17 @@ def test_phase_plan_small_cases():
     assert phase_plan(36, 10, 160) == (10, False)
     assert phase_plan(4096, 4096, 160, sink=True) == (480, False)   # 160 * (26 // 8): ~8 chunks
     assert phase_plan(1, 1, 6) == (1, True)
+
+
+@pytest.mark.parametrize("debye_waller", [False, True])
+def test_masked_records_become_plain_arrays(debye_waller):
+    """A masked structured array is taken with its mask set aside: plain arrays
+    of every site, displaced like those of the unmasked records."""
+    rec = np.zeros(6, dtype=[("atomic_number", "i"), ("x", "f"), ("y", "f"), ("z", "f"), ("occ", "f"), ("DW", "f")])
+    rec["x"], rec["y"], rec["z"], rec["atomic_number"], rec["DW"] = *np.arange(18).reshape(3, 6), 14, 0.1
+    masked = np.ma.array(rec, mask=[False] * 5 + [True])
+    a, b = (MSAGPU(200.0, 0.02, r, sampling=np.array([128, 128]), debye_waller=debye_waller, rng=np.random.RandomState(3))
+            for r in (rec, masked))
+    for name in ("supercell_xyz", "supercell_Z", "supercell_dw", "supercell_occ", "dims"):
+        u, v = getattr(a, name), getattr(b, name)
+        assert type(v) is np.ndarray and v.dtype == u.dtype and np.array_equal(u, v), name
