@@ -183,9 +183,12 @@ class FnoNet:
         self.pre = [torch.empty((C, n), **f) for _ in range(L - 1)]
         self.ga = torch.empty((C, n), **f)
         self.gb = torch.empty((C, n), **f)
-        self.hpre = self.h = self.gh = None
-        self.ones = torch.empty(n, **f)
-        call("namsa_fill", ptr(self.ones), n, np.float32(1.0), self.st)
+        self.hpre = self.h = self.gh = self.ones = None
+        if not self.head_ok(B):    # the head's hidden activation, pre-activation and gradient: its kernels keep none
+            self.hpre, self.h, self.gh = (torch.empty((Hq, n), **f) for _ in range(3))
+        if not (self.head_ok(B) and C <= 32 and self.cin <= 32):   # operand of the row sums of separate products
+            self.ones = torch.empty(n, **f)
+            call("namsa_fill", ptr(self.ones), n, np.float32(1.0), self.st)
         self._row_tables()
         self.B = B
 
@@ -214,13 +217,6 @@ class FnoNet:
     def head_ok(self, B):
         """The head's kernels of training are compiled for 32 and 64 channels and index 32 channels in 31 bits."""
         return (self.C, self.Hq) == (32, 64) and 128 * B * self.H * self.W < 2 ** 31
-
-    def _ensure_hidden(self, n):
-        """The head's hidden activation, pre-activation and gradient (the head kernels keep none)."""
-        if self.h is None or self.h.shape[1] < n:
-            torch = _torch()
-            self.hpre, self.h, self.gh = (torch.empty((self.Hq, n), dtype=torch.float32, device=self.device)
-                                          for _ in range(3))
 
     def _row_tables(self):
         """The row DFT in bf16, [Wp][2m] and transposed, zero from row W on."""
@@ -332,7 +328,6 @@ class FnoNet:
             call("namsa_fno_head", ptr(self.xs[L]), self._p("Q1"), self._p("bq1"), self._p("Q2"), self._p("bq2"), n,
                  ptr(self.out), self.st)
             return self.out
-        self._ensure_hidden(n)
         self._gemm(self._p("Q1"), (0, C, 1), ptr(self.xs[L]), (0, n, 1), ptr(self.h), (0, n, 1), Hq, n, C,
                    bias=self._p("bq1"), bias_mode=1, gelu=True, P=ptr(self.hpre))
         self._gemm(self._p("Q2"), (0, Hq, 1), ptr(self.h), (0, n, 1), ptr(self.out), (0, n, 1), 2, n, Hq,
@@ -412,13 +407,14 @@ class FnoNet:
         C2 = 2 * C
         sp = self._split(n)
         call("namsa_fill", ptr(self.grad), self.n_params, np.float32(0.0), self.st)
-        go, ones = ptr(self.gout), ptr(self.ones)
+        go = ptr(self.gout)
         ga, gb = self.ga, self.gb
         if self.head_ok(B):
             call("namsa_fno_head_backward", ptr(self.xs[L]), self._p("Q1"), self._p("bq1"), self._p("Q2"), go, n,
                  ptr(ga), self._g("Q1"), self._g("bq1"), self._g("Q2"), self._g("bq2"), self.st)
         else:
             self._gemm(go, (0, n, 1), ptr(self.h), (0, 1, n), self._g("Q2"), (0, Hq, 1), 2, Hq, n, split=sp)
+            ones = ptr(self.ones)
             self._gemm(go, (0, n, 1), ones, (0, 1, 0), self._g("bq2"), (0, 1, 1), 2, 1, n, split=sp)
             self._gemm(self._p("Q2"), (0, 1, Hq), go, (0, n, 1), ptr(self.gh), (0, n, 1), Hq, n, 2)
             call("namsa_gelu_backward", ptr(self.gh), ptr(self.hpre), Hq * n, self.st)
