@@ -57,6 +57,12 @@ int namsa_fft_supported(int n);
  * per run (namsa/cuda_kernels.py:8-56); here every length has several
  * precompiled schedules and the autotuner (namsa_amd/autotune.py) picks one.
  * The selection is process-wide; change it between launches, not during them.
+ * A schedule names a transform and the kernel that production launches run it
+ * in.  Some entries run the same transform, with the same results, in another
+ * form where the launch's size favours it: column entries in narrower strips
+ * for a few images (128, 192, 256, 512, 768, 1024), in a persistent form where
+ * the images fill it evenly (192, 256), and the 128 row entry without its
+ * prefetch beyond a workgroup per CU.
  *   namsa_sched_count  number of schedules (0 for an unsupported length)
  *   namsa_sched_name   name of schedule v, or NULL
  *   namsa_sched_get    selected schedule, or a negative status

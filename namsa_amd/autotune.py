@@ -6,7 +6,9 @@ prefetch, non-temporal traffic; see namsa_amd/csrc/passes_n.hip).  ``tune``
 times each schedule on the caller's batch shape with HIP events on the
 current stream, keeps the fastest, and records the choice in a JSON cache
 keyed by device name and transform length, so later processes start from the
-tuned schedule (``apply_cache``).
+tuned schedule (``apply_cache``).  What is timed is the form the schedule takes
+at that batch (see namsa_sched_set in namsa_hip.h): at the production group of
+128^2 ``e8.r844.pf`` runs without its prefetch, as ``e8.r844`` does.
 
     from namsa_amd import autotune
     best = autotune.tune(512, batch=4096)     # {'row': name, 'col': name, ...}

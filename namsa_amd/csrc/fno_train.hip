@@ -225,9 +225,9 @@ int launch_rows(const RowArgs& g, hipStream_t st) {
 // ------------------------------------------------------------------ the head
 // out = Q2 gelu(Q1 x + bq1) + bq2, 32 -> 64 -> 2 channels, and its gradients.
 // The hidden activation, 64 floats a pixel, is never stored: the backward pass
-// forms it again from x, 12 MFLOP of matrix products for each 118 MB (16 images
-// of 170 x 170) that hidden value, pre-activation and gradient took each time
-// they were written or read.  At that size, as products of their own -> here:
+// forms it again from x, 1.9 GFLOP of matrix products (16 images of 170 x 170;
+// 2 us at the bf16 rate) for each 118 MB (23 us) that hidden value,
+// pre-activation and gradient took each time they were written or read.  At that size, as products of their own -> here:
 // forward 129 -> 32 us, backward 340 -> 80 us, and 355 MB less held.
 
 constexpr int kHid = 64;

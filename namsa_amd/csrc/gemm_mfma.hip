@@ -377,8 +377,9 @@ __global__ void __launch_bounds__(256) gemm_split_kernel(GemmArgs g, int k_per, 
   }
 }
 
-// Pointwise layers: few rows and a short K (M <= 32 MT, K <= 16 KS) over a
-// long unit-stride N, the pixels of a batch.  Bound by streaming B and C once
+// Pointwise layers of networks of other widths than the row and head kernels
+// of training are compiled for: few rows and a short K (M <= 32 MT, K <= 16 KS)
+// over a long unit-stride N, the pixels of a batch.  Bound by streaming B and C once
 // (a tile staged through LDS wrote its bf16 operands two bytes at a time and
 // had nothing in flight across its barriers).  A wavefront holds A in the MFMA
 // layout and takes PB blocks of 32 columns, every read of B issued before the

@@ -648,8 +648,11 @@ int launch_row(int op, const RowArgs& a, hipStream_t st) {
 // per CU, twice the workgroups with half the lines to wait for are faster
 // (slice step of one image: 192^2 10.3 -> 9.4 us, 256^2 9.4 -> 8.2, 512^2 10.8
 // -> 9.6, 1024^2 20.1 -> 17.5; at two tasks per CU the two are equal or the
-// wide one is ahead).  Same operations per column: the bits do not depend on
-// it, as long as both read the propagator the same way (PG).
+// wide one is ahead).  Not at 384^2, where they gain 1% at one image (12.4 ->
+// 12.2 us) and lose from four on (12.7 and 13.0; 8 images 14.5 and 15.6), nor at
+// 2048^2, where one image's band already is 341 strips.  Same operations per
+// column: the bits do not depend on it, as long as both read the propagator
+// the same way (PG).
 //
 // Even: the same transform in a persistent form (a workgroup keeps its strip
 // and runs through images), which PROP launches take that give its resident
